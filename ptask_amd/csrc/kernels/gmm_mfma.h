@@ -1,24 +1,39 @@
-// gmm_mfma.h -- GmmAccumulate with its dense parts on the matrix cores (v_mfma_f32_16x16x4f32,
-// and v_mfma_f32_32x32x2f32 for the M-step when its moments fill four 32 x 32 tiles).
+// gmm_mfma.h -- GmmAccumulate with its products on the matrix cores (v_mfma_f32_16x16x4f32), every
+// operand in registers.
 //
 //   GmmAccumulateMfma(const float* X, GMM_DIMS d, const double* model, double* partials)
 //     Same arguments, partial-row format and tile-to-row assignment as GmmAccumulate
 //     (gmm_body.h), so GmmFinalize and every caller are unchanged; only the rounding differs.
 //
-// Per 128-point tile, with coordinates centred on g (the mean of the component means, one
-// per-dimension vector per launch: x' = x - g, c'_k = mu_k - g):
-//   E-step  the squared Mahalanobis distances of all points to all components as one product
-//           [x'^2 | x'] (128 x 2Dp)  .  [iv ; -2 iv c'] (2Dp x Kp)  + sum_m iv c'^2,
-//           then log responsibilities lp = C_k - d/2 and the per-point log-sum-exp on the VALU.
-//           The expansion cancels (|x'|^2 iv against the distance); it runs only while every
-//           reciprocal variance is at most GMM_MFMA_IV_LIMIT.  Otherwise (the first EM step,
-//           var = 1e-10) the block keeps GmmAccumulate's per-component differences on the VALU.
-//   M-step  the moments about g as one product  R^T (Kp x 128) . [x' | x'^2] (128 x 2Dp);
-//           W_k = sum_p R_pk on the VALU.  Tile sums are binary32 (in MFMA order), added into
-//           binary64 per block, and converted once per block to moments about the table centres
-//           c = mu_k:  su = A1 - c' W,  suu = A2 - 2 c' A1 + c'^2 W  (binary64).
-// Output tile ownership is fixed per wave, so each partial row is a fixed function of (N,
-// blocks): bitwise reproducible run to run.
+// A wave works alone on groups of 16 points, with coordinates centred on g (the mean of the
+// component means, one per-dimension vector per launch: x' = x - g, c'_k = mu_k - g):
+//   E-step  the squared Mahalanobis distances of its 16 points to all components as one product
+//           [x'^2 | x'] (16 x 2W) . [iv ; -2 iv c'] (2W x Kp)  + sum_m iv c'^2.  The right-hand
+//           operand is the same for every point: it stays in registers for the whole launch.
+//   log-sum-exp  of each point, in the product's own output layout: lane (l4, l16) holds points
+//           4 l4 + r (r < 4) against components 16 kt + l16, so a point's components are a few
+//           registers of the 16 lanes of one DPP row.  Base 2 throughout.
+//   M-step  the moments about g as one product  R^T (Kp x 16) . [x' | x'^2] (16 x 2W).  The
+//           responsibilities are its left operand exactly as the E-step leaves them: lane (l4,
+//           l16) supplies A[component l16][point 4 l4 + r], one product per r (which four points
+//           form a product's inner dimension is free, as long as both operands agree).
+// So nothing passes through LDS between the products and no wave waits for another.
+//
+// The expansion in the E-step cancels (|x'|^2 iv against the distance); it runs only while every
+// reciprocal variance is at most GMM_MFMA_IV_LIMIT.  Otherwise (the first EM step, var = 1e-10) the
+// block runs GmmAccumulate's body.
+//
+// Sums are binary32 over at most 128 points of one wave (in MFMA order), then binary64 (LDS for the
+// block, or registers where the moments are few), converted once per block to moments about the
+// table centres c = mu_k:  su = A1 - c' W,  suu = A2 - 2 c' A1 + c'^2 W.  The order of every sum is
+// a fixed function of (N, blocks): bitwise reproducible run to run.
+//
+// Bound: the matrix cores (8 N D K flops per step; 32 cycles of a SIMD per product).  Two waves per
+// SIMD (at most 256 registers) cover each other's log-sum-exp, about a quarter of the products'
+// issue time at D = 32, K = 64.  Measured there with N = 2M, 768 blocks: 328 us per launch, the matrix
+// cores busy 66% of the time; 612 us when tiles of coordinates and responsibilities passed through
+// LDS between the products (four barriers a tile, an LDS read per operand).  N = 50,001, D = 16, K = 24
+// (one tile per block): 13.5 us, 27.8 before, when every block first built the operand in LDS.
 #pragma once
 
 #include "gmm_body.h"
@@ -26,298 +41,358 @@
 typedef float gmm_f4 __attribute__((ext_vector_type(4)));
 
 #define GMM_MFMA_IV_LIMIT 1.0e3f
-#define MXS (DMAX + 4)  // floats per point row of centred coordinates
-#define MRS (KMAX + 5)  // floats per point row of (log) responsibilities: odd, so a wave reading
-                        // one component of 64 points hits distinct banks
-#define MBS (KMAX + 4)  // floats per row of the E-step B operand
+#define GMM_GROUP 16  // points per wave and product
+// doubles per component row of the block's moment sums (2 W moments): the four rows a wave's store
+// touches then start 32 banks apart
+#define GMM_ACC_STRIDE(W) (2 * (W) + 4)
 
 struct GmmMfmaShared {
     union {
-        struct {
-            float sX[TILE * MXS];
-            float sR[TILE * MRS];
-        } t;
-        double sAcc[KMAX * 2 * DMAX];  // the block's moment sums about g, after the last tile
+        GmmShared valu;                                // the steps before the E-step expansion is safe
+        double acc[KMAX * GMM_ACC_STRIDE(DMAX)];       // the block's moment sums about g
     } u;
-    float sB[2 * DMAX * MBS];
-    float sE[KMAX];
-    float sG[DMAX];
-    float sMax[2][TILE];
-    float sSum[2][TILE];
-    float sWp[4][KMAX];  // per-wave column sums of a tile's responsibilities
-    double sW[KMAX];
-    double sLL[4];
+    float g[DMAX];
+    double w[4][KMAX];
+    double ll[4];
+    unsigned turn;  // additions to acc made so far by the block's waves
 };
 
-// E-step products of component tile kt with point tiles IL pg .. IL pg + IL - 1 of the tile in
-// sX: IL independent MFMA chains, interleaved, sharing each B operand load; log responsibilities
-// C_k - d/2 into sR.
-template <int IL, int NC>
-__device__ __forceinline__ void gmm_mfma_estep(GmmMfmaShared &sh, const float *__restrict__ sX, float *__restrict__ sR,
-                                               int kt, int pg, int K, int l16, int l4) {
-#pragma clang fp contract(fast)
-    constexpr int Dp = 4 * NC, D2 = 2 * Dp;
-    const float *bb = sh.sB + kt * 16 + l16;
-    gmm_f4 acc[IL];
-#pragma unroll
-    for (int u = 0; u < IL; ++u) acc[u] = gmm_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D2 / 4; ++s) {
-        const int c = 4 * s + l4, cx = c < Dp ? c : c - Dp;
-        const float bv = bb[c * MBS];
-#pragma unroll
-        for (int u = 0; u < IL; ++u) {
-            const float xv = sX[((IL * pg + u) * 16 + l16) * MXS + cx];
-            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(c < Dp ? xv * xv : xv, bv, acc[u], 0, 0, 0);
-        }
-    }
-    const int k = kt * 16 + l16;
-    if (k < K) {
-        const float e = sh.sE[k];
-#pragma unroll
-        for (int u = 0; u < IL; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sR[((IL * pg + u) * 16 + 4 * l4 + r) * MRS + k] = fmaf(-0.5f, acc[u][r], e);
-    }
+// Max and sum of four values over the 16 lanes of a DPP row; every lane gets the results.  Rotating
+// by 8, 4, 2 and 1 the four chains are interleaved, so an operand is always three instructions old
+// (a DPP operand may be read two after it is written): written as instructions because the
+// compiler takes the chains one after the other with a wait and a move per step.
+#define GMM_DPP4(OP, N)                                              \
+    OP " %0, %0, %0 row_ror:" N " row_mask:0xf bank_mask:0xf\n\t"    \
+    OP " %1, %1, %1 row_ror:" N " row_mask:0xf bank_mask:0xf\n\t"    \
+    OP " %2, %2, %2 row_ror:" N " row_mask:0xf bank_mask:0xf\n\t"    \
+    OP " %3, %3, %3 row_ror:" N " row_mask:0xf bank_mask:0xf\n\t"
+#define GMM_ROW4(OP) "s_nop 1\n\t" GMM_DPP4(OP, "8") GMM_DPP4(OP, "4") GMM_DPP4(OP, "2") GMM_DPP4(OP, "1")
+__device__ __forceinline__ void gmm_row_max4(float (&v)[4]) {
+    asm(GMM_ROW4("v_max_f32_dpp") : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+__device__ __forceinline__ void gmm_row_sum4(float (&v)[4]) {
+    asm(GMM_ROW4("v_add_f32_dpp") : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
 }
 
-template <int NC>
-__device__ __forceinline__ void gmm_mfma_tiles(const float *__restrict__ X, const GMM_DIMS &d,
+// One partial row.  W = 8 DC dimensions (D rounded up to 8), KT component tiles of 16.  Returns
+// false, having written nothing, when the E-step expansion is not safe (uniform over the block).
+template <int DC, int KT>
+__device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, const GMM_DIMS &d,
                                                const double *__restrict__ model, double *__restrict__ row,
                                                long long t0, long long t1, long long tstep, GmmMfmaShared &sh) {
 #pragma clang fp contract(fast)
-    float *sX = sh.u.t.sX, *sR = sh.u.t.sR;
-    const int D = d.D, K = d.K, Dp = 4 * NC, D2 = 2 * Dp, Kp = (K + 15) & ~15;
-    const int KT = Kp >> 4, JT = (D2 + 15) >> 4;
-    // M-step on 32 x 32 x 2 products when the moments fill four 32 x 32 tiles (K and 2 Dp in
-    // (32, 64]): one tile per wave, half the operand reads per flop of the 16 x 16 x 4 form
-    const int JT2 = (D2 + 31) >> 5;
-    const bool m32 = ((K + 31) >> 5) * JT2 == 4;
-    typedef float gmm_f16 __attribute__((ext_vector_type(16)));
-    const int tid = threadIdx.x, lane = tid & 63;
+    constexpr int W = 8 * DC, NF = 2 * DC;            // dimensions; dimensions per lane of the E-step
+    constexpr int JT = DC;                            // 16-wide tiles of the 2 W moments
+    constexpr int NS = W % 16 == 0 ? JT / 2 : JT;     // coordinate registers per point of the M-step
+    constexpr bool kRegAcc = KT * JT <= 4;            // binary64 sums in registers
+    constexpr int kStride = GMM_ACC_STRIDE(W);
+    constexpr float kLog2e = 1.44269504088896340736f;
+    const int D = d.D, K = d.K, Dp = ptk_gmm_dpad(&d);
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, l4 = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l16 = lane & 15, l4 = lane >> 4;
     const float *__restrict__ tab = (const float *)(model + ptk_gmm_table(&d));
-    const float *__restrict__ Cf = tab + 2 * K * Dp;
 
-    // ---- per launch: centre, E-step operand and constants
-    for (int m = tid; m < Dp; m += 256) {
-        double s = 0;
-        for (int k = 0; k < K; ++k) s += (double)tab[2 * k * Dp + m];
-        sh.sG[m] = m < D ? (float)(s / K) : 0.f;
-    }
-    __syncthreads();
+    // ---- per launch: the centre and the E-step operand of this lane's dimensions f0 .. f0 + NF - 1
+    const int f0 = l4 * NF;
+    float g[NF], b1[KT][NF], b2[KT][NF], ek[KT];
     bool big = false;
-    for (int i = tid; i < D2 * Kp; i += 256) {
-        const int c = i / Kp, k = i - c * Kp;
-        float v = 0.f;
-        if (k < K) {
-            const int m = c < Dp ? c : c - Dp;
-            const float iv = tab[2 * k * Dp + Dp + m];
-            if (m < D && !(iv <= GMM_MFMA_IV_LIMIT)) big = true;
-            v = c < Dp ? iv : -2.f * iv * (tab[2 * k * Dp + m] - sh.sG[m]);
+    {
+        double s[NF];
+#pragma unroll
+        for (int i = 0; i < NF; ++i) s[i] = 0;
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+            const int k = kt * 16 + l16;
+#pragma unroll
+            for (int i = 0; i < NF; ++i) {
+                const bool on = k < K && f0 + i < D;
+                const float *e = tab + 2 * (k < K ? k : 0) * Dp + (f0 + i < D ? f0 + i : 0);
+                const float mu = e[0], iv = e[Dp];
+                b1[kt][i] = on ? mu : 0.f;
+                b2[kt][i] = on ? iv : 0.f;
+                if (on && !(iv <= GMM_MFMA_IV_LIMIT)) big = true;
+                s[i] += (double)b1[kt][i];
+            }
         }
-        sh.sB[c * MBS + k] = v;
+        if (__any(big)) return false;
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) s[i] += __shfl_xor(s[i], off, 64);
+            g[i] = (float)(s[i] / K);  // 0 for i past D
+        }
+        if (wv == 0 && l16 == 0)
+#pragma unroll
+            for (int i = 0; i < NF; ++i) sh.g[f0 + i] = g[i];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+            const int k = kt * 16 + l16;
+            double q = 0;
+#pragma unroll
+            for (int i = 0; i < NF; ++i) {
+                const float mu = b1[kt][i], iv = b2[kt][i];
+                const double cp = (double)mu - (double)g[i];
+                q += (double)iv * cp * cp;
+                b1[kt][i] = -2.f * iv * (mu - g[i]);
+            }
+            q += __shfl_xor(q, 16, 64);
+            q += __shfl_xor(q, 32, 64);
+            // log2 of the responsibilities: a component past the last gets weight 0
+            ek[kt] = k < K ? (float)(((double)tab[2 * K * Dp + k] - 0.5 * q) * 1.44269504088896340736) : -INFINITY;
+        }
     }
-    for (int k = tid; k < K; k += 256) {
-        double q = 0;
-        for (int m = 0; m < D; ++m) {
-            const double cp = (double)tab[2 * k * Dp + m] - (double)sh.sG[m];
-            q += (double)tab[2 * k * Dp + Dp + m] * cp * cp;
-        }
-        sh.sE[k] = (float)((double)Cf[k] - 0.5 * q);
-    }
-    const bool mfmaE = !__syncthreads_or(big);
-
-    // E-phase ownership of the VALU fallback and of the log-sum-exp: point ep, components of half eh
-    const int ep = (wv & 1) * 64 + lane, eh = wv >> 1;
-    const int kh = (K + 1) >> 1, k0 = eh * kh, k1 = min(K, k0 + kh);
-
-    double dacc[4][4];
+    for (int i = tid; i < KT * 16 * kStride; i += 256) sh.u.acc[i] = 0;
+    if (tid == 0) sh.turn = 0;
+    __syncthreads();
+    // ---- the M-step's coordinates of this lane: moment column 16 jt + l16 is dimension jd of point
+    // 4 l4 + r, squared from column W on
+    int jd[NS];
+    float gm[NS];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dacc[q][r] = 0;
-    double aw = 0, ll = 0;
-
-    // next tile's coordinates in registers while the current one computes (gmm_fetch_tile)
-    float pf[2 * NC];
-    gmm_fetch_tile<NC>(X, d, t0, t1, pf);
-    for (long long t = t0; t < t1; t += tstep) {
-        const long long p0 = t * TILE;
-        const int np = (int)min((long long)TILE, (long long)d.N - p0);
-        const float *__restrict__ xt = X + p0 * D;
-#pragma unroll
-        for (int j = 0; j < 2 * NC; ++j) {
-            const int i = tid + 256 * j, p = i / Dp, m = i - p * Dp;
-            sX[p * MXS + m] = (p < np && m < D) ? pf[j] - sh.sG[m] : 0.f;
-        }
-        __syncthreads();
-        gmm_fetch_tile<NC>(X, d, t + tstep, t1, pf);
-
-        // ---- E-step: log responsibilities into sR[p][k]
-        if (mfmaE) {
-            // job jb: component tile jb % KT against point tiles 4 (jb / KT) .. +3, four
-            // independent MFMA chains interleaved (enough to cover the product's latency)
-            for (int jb = wv; jb < 2 * KT; jb += 4) gmm_mfma_estep<4, NC>(sh, sX, sR, jb % KT, jb / KT, K, l16, l4);
-        } else {
-            // differences to each component mean from the point itself, as GmmAccumulate
-            float x[4 * NC];
-#pragma unroll
-            for (int m = 0; m < 4 * NC; ++m) x[m] = (ep < np && m < D) ? xt[(long long)ep * D + m] : 0.f;
-            for (int k = k0; k < k1; ++k) {
-                const float *__restrict__ tk = tab + 2 * k * Dp;
-                float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    const float4 mu = *(const float4 *)(tk + 4 * c);
-                    const float4 iv = *(const float4 *)(tk + Dp + 4 * c);
-                    const float u0 = x[4 * c] - mu.x, u1 = x[4 * c + 1] - mu.y;
-                    const float u2 = x[4 * c + 2] - mu.z, u3 = x[4 * c + 3] - mu.w;
-                    s0 = fmaf(u0 * u0, iv.x, s0);
-                    s1 = fmaf(u1 * u1, iv.y, s1);
-                    s0 = fmaf(u2 * u2, iv.z, s0);
-                    s1 = fmaf(u3 * u3, iv.w, s1);
-                }
-                sR[ep * MRS + k] = fmaf(-0.5f, s0 + s1, Cf[k]);
-            }
-        }
-        __syncthreads();
-
-        // ---- per-point log-sum-exp, responsibilities, log-likelihood
-        float mx = -INFINITY;
-#pragma unroll 8
-        for (int k = k0; k < k1; ++k) mx = fmaxf(mx, sR[ep * MRS + k]);
-        sh.sMax[eh][ep] = mx;
-        __syncthreads();
-        mx = fmaxf(sh.sMax[0][ep], sh.sMax[1][ep]);
-        float sum = 0.f;
-#pragma unroll 8
-        for (int k = k0; k < k1; ++k) sum += __expf(sR[ep * MRS + k] - mx);
-        sh.sSum[eh][ep] = sum;
-        __syncthreads();
-        const float tmp = mx + __logf(sh.sSum[0][ep] + sh.sSum[1][ep]);
-        const bool valid = ep < np;
-#pragma unroll 8
-        for (int k = k0; k < k1; ++k) sR[ep * MRS + k] = valid ? __expf(sR[ep * MRS + k] - tmp) : 0.f;
-        if (valid && eh == 0) ll += (double)tmp;
-        __syncthreads();
-
-        // ---- M-step: R^T [x' | x'^2] on the matrix cores, W on the VALU.
-        if (m32) {
-            // wave wv: components 32 (wv / JT2) .., features 32 (wv % JT2) ..; lane l supplies
-            // A[l % 32][l / 32] = R[p][k] and B[l / 32][l % 32] = [x' | x'^2][p][j] for the two
-            // points p = 2s + l / 32 of step s; D[8(r/4) + 4(l/32) + r%4][l % 32] in acc[r]
-            const int kt2 = wv / JT2, jt2 = wv - kt2 * JT2, l32 = lane & 31, h = lane >> 5;
-            const int ki = kt2 * 32 + l32, j = jt2 * 32 + l32;
-            const bool rowok = ki < K, jlo = j < Dp, jhi = j >= Dp && j < D2;
-            const int jx = j < Dp ? j : (j < D2 ? j - Dp : 0);
-            gmm_f16 acc = {};
-#pragma unroll 8
-            for (int s = 0; s < TILE / 2; ++s) {
-                const int p = 2 * s + h;
-                const float a = rowok ? sR[p * MRS + ki] : 0.f;
-                const float xv = sX[p * MXS + jx];
-                const float b = jlo ? xv : (jhi ? xv * xv : 0.f);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dacc[q][r] += (double)acc[4 * q + r];
-        } else {
-            // the wave's four 16 x 16 output tiles (tt = wv + 4q) accumulated together, their
-            // products interleaved; a tile past the last (tt >= KT JT) multiplies zeros and is
-            // not stored
-            int ki[4], jx[4];
-            bool rowok[4], jlo[4], jhi[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int tt = wv + 4 * q;
-                const bool on = tt < KT * JT;
-                const int kt = on ? tt / JT : 0, jt = on ? tt - kt * JT : 0;
-                const int j = jt * 16 + l16;
-                ki[q] = kt * 16 + l16;
-                rowok[q] = on && ki[q] < K;
-                jlo[q] = on && j < Dp;
-                jhi[q] = on && j >= Dp && j < D2;
-                jx[q] = j < Dp ? j : (j < D2 ? j - Dp : 0);
-            }
-            gmm_f4 acc[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] = gmm_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-            for (int s = 0; s < TILE / 4; ++s) {
-                const int p = 4 * s + l4;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float a = rowok[q] ? sR[p * MRS + ki[q]] : 0.f;
-                    const float xv = sX[p * MXS + jx[q]];
-                    const float b = jlo[q] ? xv : (jhi[q] ? xv * xv : 0.f);
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[q], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (wv + 4 * q < KT * JT)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) dacc[q][r] += (double)acc[q][r];
-        }
-        {   // W: wave wv sums points [32 wv, 32 wv + 32) of component `lane`; the four wave sums
-            // are added in wave order below, after the barrier
-            float w = 0.f;
-            if (lane < K) {
-#pragma unroll 8
-                for (int p = 32 * wv; p < 32 * wv + 32; ++p) w += sR[p * MRS + lane];
-            }
-            sh.sWp[wv][lane] = w;
-        }
-        __syncthreads();
-        if (tid < K) aw += (double)(((sh.sWp[0][tid] + sh.sWp[1][tid]) + sh.sWp[2][tid]) + sh.sWp[3][tid]);
+    for (int j = 0; j < NS; ++j) {
+        const int c = 16 * j + l16, m = c < W ? c : c - W;
+        jd[j] = m < D ? m : D - 1;  // a column past D is never read back
+        gm[j] = sh.g[m];
     }
 
-    // ---- the block's moments about the table centres, one partial row
-    double *sAcc = sh.u.sAcc;
-    if (m32) {
-        const int kt2 = wv / JT2, jt2 = wv - kt2 * JT2, j = jt2 * 32 + (lane & 31);
+    gmm_f4 acc[KT][JT];
+    double dacc[kRegAcc ? KT : 1][kRegAcc ? JT : 1][4];
+    float w[KT];
+    double dw[KT], ll = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+    for (int kt = 0; kt < KT; ++kt) {
+        w[kt] = 0.f;
+        dw[kt] = 0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int k = kt2 * 32 + 8 * q + 4 * (lane >> 5) + r;
-                if (k < K && j < D2) sAcc[k * D2 + j] = dacc[q][r];
-            }
-    } else {
+        for (int jt = 0; jt < JT; ++jt) {
+            acc[kt][jt] = gmm_f4{0.f, 0.f, 0.f, 0.f};
+            if (kRegAcc)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int tt = wv + 4 * q;
-            if (tt < KT * JT) {
-                const int kt = tt / JT, jt = tt - kt * JT, j = jt * 16 + l16;
+                for (int r = 0; r < 4; ++r) dacc[kt][jt][r] = 0;
+        }
+    }
+    // this wave's binary32 sums (at most 128 points) into the binary64 ones
+    auto *lacc = (__attribute__((address_space(3))) double *)sh.u.acc;
+    auto *lturn = (__attribute__((address_space(3))) unsigned *)&sh.turn;
+    auto flush = [&]() {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+            dw[kt] += (double)w[kt];
+            w[kt] = 0.f;
+#pragma unroll
+            for (int jt = 0; jt < JT; ++jt) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int k = kt * 16 + 4 * l4 + r;
-                    if (k < K && j < D2) sAcc[k * D2 + j] = dacc[q][r];
+                    if (kRegAcc) dacc[kt][jt][r] += (double)acc[kt][jt][r];
+                    else __builtin_amdgcn_ds_atomic_fadd_f64(lacc + (16 * kt + 4 * l4 + r) * kStride + 16 * jt + l16,
+                                                             (double)acc[kt][jt][r]);
                 }
+                acc[kt][jt] = gmm_f4{0.f, 0.f, 0.f, 0.f};
             }
         }
+    };
+
+    // Wave wv takes points [32 wv, 32 wv + 32) of each 128-point tile, as two groups: group n of the
+    // wave is points 16 (n & 1) .. of tile t0 + (n >> 1) tstep.  A group's coordinates are loaded
+    // while the group before it computes, through a buffer that ends with the last point: what lies
+    // past it reads as 0 (such a point gets responsibility 0; a dimension past D is multiplied by 0
+    // or never read back), so a group is always the same loads, whatever D and its alignment.
+    float xe[NF], xm[NS][4];
+    auto base = [&](long long t, int q) { return t * TILE + 32 * wv + 16 * q; };
+    auto group = [&](long long p0) {
+        const long long left = ((long long)d.N - p0) * D * 4;
+        const int bytes = left < 0 ? 0 : (int)min(left, (long long)GMM_GROUP * DMAX * 4);
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(X + (left > 0 ? p0 * D : 0)), (short)0, bytes, 0x00020000);
+    };
+    const int oe = (l16 * D + f0) * 4;
+    int om[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) om[j] = (4 * l4 * D + jd[j]) * 4;
+    auto loadE = [&](long long p0) {
+        const auto rs = group(p0);
+        constexpr int V = NF % 4 == 0 ? 4 : 2;
+#pragma unroll
+        for (int c = 0; c < NF; c += V) {
+            if (V == 4) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, oe + 4 * c, 0, 0);
+#pragma unroll
+                for (int i = 0; i < V; ++i) xe[c + i] = __builtin_bit_cast(float, (unsigned)v[i]);
+            } else {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, oe + 4 * c, 0, 0);
+#pragma unroll
+                for (int i = 0; i < V; ++i) xe[c + i] = __builtin_bit_cast(float, (unsigned)v[i]);
+            }
+        }
+    };
+    auto loadM = [&](long long p0) {
+        const auto rs = group(p0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < NS; ++j)
+                xm[j][r] = __builtin_bit_cast(float, (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rs, om[j] + 4 * r * D, 0, 0));
+    };
+    int turn = 0;  // tiles of this wave so far
+    if (t0 < t1) {
+        loadE(base(t0, 0));
+        loadM(base(t0, 0));
     }
-    if (tid < K) sh.sW[tid] = aw;
+    for (long long t = t0; t < t1; t += tstep) {
+#pragma unroll 1
+        for (int q = 0; q < 2; ++q) {
+            const long long p0 = base(t, q);
+            const long long pn = q == 0 ? base(t, 1) : t + tstep < t1 ? base(t + tstep, 0) : p0;
+            const int np = (int)min((long long)GMM_GROUP, d.N - p0);  // valid points (<= 0: none)
+            // ---- E-step
+            float a1[NF], a2[NF];
+#pragma unroll
+            for (int i = 0; i < NF; ++i) {
+                a1[i] = xe[i] - g[i];
+                a2[i] = a1[i] * a1[i];
+            }
+            loadE(pn);
+            gmm_f4 e[KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) e[kt] = gmm_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NF; ++i)
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt)
+                    e[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[i], b2[kt][i], e[kt], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NF; ++i)
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt)
+                    e[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[i], b1[kt][i], e[kt], 0, 0, 0);
+            // ---- log-sum-exp of point 4 l4 + r over the row's lanes; responsibilities into e
+            float mx[4], sum[4], lse[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                mx[r] = -INFINITY;
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    e[kt][r] = fmaf(-0.5f * kLog2e, e[kt][r], ek[kt]);
+                    mx[r] = kt == 0 ? e[kt][r] : fmaxf(mx[r], e[kt][r]);
+                }
+            }
+            gmm_row_max4(mx);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    e[kt][r] = __builtin_amdgcn_exp2f(e[kt][r] - mx[r]);
+                    sum[r] = kt == 0 ? e[kt][r] : sum[r] + e[kt][r];
+                }
+            gmm_row_sum4(sum);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float inv = 4 * l4 + r < np ? __builtin_amdgcn_rcpf(sum[r]) : 0.f;
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    e[kt][r] *= inv;
+                    w[kt] += e[kt][r];
+                }
+                lse[r] = mx[r] + __builtin_amdgcn_logf(sum[r]);
+            }
+            {   // the sixteen lanes of a row hold the same four values: lane l16 = r adds point r's
+                const float v = l16 == 0 ? lse[0] : l16 == 1 ? lse[1] : l16 == 2 ? lse[2] : lse[3];
+                if (l16 < 4 && 4 * l4 + l16 < np) ll += (double)v;
+            }
+            // ---- M-step
+            float x1[NS][4], x2[NS][4];
+#pragma unroll
+            for (int j = 0; j < NS; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    x1[j][r] = xm[j][r] - gm[j];
+                    x2[j][r] = x1[j][r] * x1[j][r];
+                }
+            loadM(pn);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int jt = 0; jt < JT; ++jt) {
+                    const float b = NS == JT ? (16 * jt + l16 < W ? x1[jt % NS][r] : x2[jt % NS][r])
+                                    : jt < NS ? x1[jt % NS][r] : x2[jt % NS][r];
+#pragma unroll
+                    for (int kt = 0; kt < KT; ++kt)
+                        acc[kt][jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[kt][r], b, acc[kt][jt], 0, 0, 0);
+                }
+        }
+        // every fourth tile of the wave.  The waves take turns at the block's sums in tile order, so
+        // that the order of the additions is fixed: turn n waits for turn n - 1, made by the wave
+        // before at its previous tile (every wave of the block counts the same tiles, so each turn
+        // comes).  A wave is held up only when another is behind by a tile; a barrier per tile would
+        // have all four wait for the slowest each time.
+        if (kRegAcc) {
+            if ((turn & 3) == 3) flush();
+        } else if ((turn & 3) == wv) {
+            while (__hip_atomic_load(lturn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != (unsigned)turn)
+                __builtin_amdgcn_s_sleep(1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            flush();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (lane == 0) __hip_atomic_store(lturn, (unsigned)turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        ++turn;
+    }
+    if (kRegAcc) flush();
     __syncthreads();
+#pragma unroll 1
+    for (int v = 0; v < 4; ++v) {  // what is left, in wave order
+        if (wv == v) {
+            if (kRegAcc) {
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                    for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            sh.u.acc[(16 * kt + 4 * l4 + r) * kStride + 16 * jt + l16] += dacc[kt][jt][r];
+            } else {
+                flush();
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+        double v = dw[kt];
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (l4 == 0) sh.w[wv][16 * kt + l16] = v;
+    }
+    ll *= 0.69314718055994530942;  // base 2 to natural
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) ll += __shfl_xor(ll, off, 64);
+    if (lane == 0) sh.ll[wv] = ll;
+    __syncthreads();
+
+    // ---- the block's moments about the table centres, one partial row
     for (int i = tid; i < K * D; i += 256) {
         const int k = i / D, m = i - k * D;
-        const double w = sh.sW[k], a1 = sAcc[k * D2 + m], a2 = sAcc[k * D2 + Dp + m];
-        const double cp = (double)tab[2 * k * Dp + m] - (double)sh.sG[m];
-        row[K + k * D + m] = a1 - cp * w;
-        row[K + K * D + k * D + m] = a2 - 2.0 * cp * a1 + cp * cp * w;
+        const double wk = sh.w[0][k] + sh.w[1][k] + sh.w[2][k] + sh.w[3][k];
+        const double a1 = sh.u.acc[k * kStride + m], a2 = sh.u.acc[k * kStride + W + m];
+        const double cp = (double)tab[2 * k * Dp + m] - (double)sh.g[m];
+        row[K + i] = a1 - cp * wk;
+        row[K + K * D + i] = a2 - 2.0 * cp * a1 + cp * cp * wk;
     }
-    if (tid < K) row[tid] = aw;
-    double v = ll;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) sh.sLL[wv] = v;
-    __syncthreads();
-    if (tid == 0) row[K + 2 * K * D] = sh.sLL[0] + sh.sLL[1] + sh.sLL[2] + sh.sLL[3];
-    __syncthreads();
+    if (tid < K) row[tid] = sh.w[0][tid] + sh.w[1][tid] + sh.w[2][tid] + sh.w[3][tid];
+    if (tid == 0) row[K + 2 * K * D] = sh.ll[0] + sh.ll[1] + sh.ll[2] + sh.ll[3];
+    __syncthreads();  // a block may go on to another unit, which reuses sh
+    return true;
+}
+
+template <int DC>
+__device__ __forceinline__ bool gmm_mfma_comps(const float *__restrict__ X, const GMM_DIMS &d,
+                                               const double *__restrict__ model, double *__restrict__ row,
+                                               long long t0, long long t1, long long ts, GmmMfmaShared &sh) {
+    switch ((d.K + 15) >> 4) {
+        case 1: return gmm_mfma_tiles<DC, 1>(X, d, model, row, t0, t1, ts, sh);
+        case 2: return gmm_mfma_tiles<DC, 2>(X, d, model, row, t0, t1, ts, sh);
+        case 3: return gmm_mfma_tiles<DC, 3>(X, d, model, row, t0, t1, ts, sh);
+        default: return gmm_mfma_tiles<DC, 4>(X, d, model, row, t0, t1, ts, sh);
+    }
 }
 
 __device__ __forceinline__ void gmm_mfma_unit(const float *__restrict__ X, const GMM_DIMS &d,
@@ -325,14 +400,12 @@ __device__ __forceinline__ void gmm_mfma_unit(const float *__restrict__ X, const
                                               int b, GmmMfmaShared &sh) {
     const long long t0 = b, t1 = ((long long)d.N + TILE - 1) / TILE, ts = d.blocks;
     double *row = partials + (long long)b * ptk_gmm_partial_stride(&d);
-    switch (ptk_gmm_dpad(&d) >> 2) {
-        case 1: gmm_mfma_tiles<1>(X, d, model, row, t0, t1, ts, sh); break;
-        case 2: gmm_mfma_tiles<2>(X, d, model, row, t0, t1, ts, sh); break;
-        case 3: gmm_mfma_tiles<3>(X, d, model, row, t0, t1, ts, sh); break;
-        case 4: gmm_mfma_tiles<4>(X, d, model, row, t0, t1, ts, sh); break;
-        case 5: gmm_mfma_tiles<5>(X, d, model, row, t0, t1, ts, sh); break;
-        case 6: gmm_mfma_tiles<6>(X, d, model, row, t0, t1, ts, sh); break;
-        case 7: gmm_mfma_tiles<7>(X, d, model, row, t0, t1, ts, sh); break;
-        default: gmm_mfma_tiles<8>(X, d, model, row, t0, t1, ts, sh); break;
+    bool done;
+    switch ((d.D + 7) >> 3) {
+        case 1: done = gmm_mfma_comps<1>(X, d, model, row, t0, t1, ts, sh); break;
+        case 2: done = gmm_mfma_comps<2>(X, d, model, row, t0, t1, ts, sh); break;
+        case 3: done = gmm_mfma_comps<3>(X, d, model, row, t0, t1, ts, sh); break;
+        default: done = gmm_mfma_comps<4>(X, d, model, row, t0, t1, ts, sh); break;
     }
+    if (!done) gmm_accumulate_unit(X, d, model, partials, b, sh.u.valu);
 }
