@@ -44,8 +44,8 @@ constexpr unsigned long long kAlign = 256;
 constexpr int kFdtdCap = 16384, kGbCap = 8192, kGmmCap = 8192;
 // device work-list lengths: FDTD tiles, FDTD instances, groupby chunk units, groupby buckets,
 // GMM accumulate units, GMM finalize units, three-step items, three-step blocks, groupby tiles,
-// groupby half buckets, groupby quarter buckets
-constexpr int kCounts = 11;
+// groupby half buckets, groupby quarter buckets, "fewer three-step tiles than blocks" (0 or 1)
+constexpr int kCounts = 12;
 
 unsigned long long Up(unsigned long long x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
@@ -417,8 +417,12 @@ size_t FdtdTiles(const ptk_batch *B, int cols, int depth) {
 // tiles of the resident instances in order, q = N / G whole-depth tiles per block taken
 // round-robin (block b: tiles b, b + G, ...; at any time the blocks stream neighbouring tiles at
 // about the same planes, so their overlap is shared in L2), then the planes of the remaining
-// tiles cut into G equal runs in (tile, plane) order, one per block.  Items are grouped by
-// block; at most N + G of them.
+// M = N - qG tiles, one segment per block.  A segment costs its planes plus the pipeline's
+// T + 2(T-1), so the remaining tiles are cut into slabs of at most L planes, the smallest L that gives
+// at most G slabs; or, where that leaves too many blocks idle, into G equal runs in (tile, plane)
+// order, most of which cross from one tile into the next and pay the pipeline twice (as
+// FdtdThreeStepPersistent cuts its own).  24 instances of edge 16..40 (252 slabs of at most 11
+// planes; runs of 9.3, of which two in three straddled): 29 us per launch against 40.  Items are grouped by block; at most N + G of them.
 void BuildSchedule3(ptk_batch *B, const std::vector<int4> &t3, int G) {
     const size_t N = t3.size(), q = N / (size_t)G;
     long long W = 0;
@@ -426,11 +430,41 @@ void BuildSchedule3(ptk_batch *B, const std::vector<int4> &t3, int G) {
     size_t idx = q * (size_t)G;  // first remaining tile whose planes reach past `pos`
     long long pos = 0;          // planes of the remaining tiles before tile idx
     B->tiles3.n = 0;
+    // slabs of at most L planes: `total` of them, slab j on block j G / total
+    constexpr int kPipe = 3 + 2 * (3 - 1);
+    int L = 0;
+    long long total = 0;
+    if (idx < N) {
+        auto slabsOf = [&](int planes) {
+            long long c = 0;
+            for (size_t i = idx; i < N; ++i) c += (t3[i].w + planes - 1) / planes;
+            return c;
+        };
+        int lo = 1, hi = 1;
+        for (size_t i = idx; i < N; ++i) hi = std::max(hi, t3[i].w);  // one slab per tile: M < G of them
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (slabsOf(mid) <= G) hi = mid;
+            else lo = mid + 1;
+        }
+        if (lo + kPipe <= W / G + 2 * kPipe) L = lo, total = slabsOf(lo);
+    }
+    size_t tile = idx;        // the next slab: slab `part` of this tile, number `slab` in all
+    long long part = 0, slab = 0;
     for (int b = 0; b < G; ++b) {
         B->t3start.host[b] = (int)B->tiles3.n;
         for (size_t r = 0; r < q; ++r) {
             const int4 &t = t3[r * (size_t)G + (size_t)b];
             B->tiles3.host[B->tiles3.n++] = int4{t.x, t.y, t.z, 0 | (t.w << 16)};
+        }
+        if (L) {
+            for (; slab < total && slab * G / total == b; ++slab) {  // none or one
+                const int4 &t = t3[tile];
+                const long long c = (t.w + L - 1) / L, k0 = t.w * part / c, k1 = t.w * (part + 1) / c;
+                B->tiles3.host[B->tiles3.n++] = int4{t.x, t.y, t.z, (int)k0 | ((int)k1 << 16)};
+                if (++part == c) ++tile, part = 0;
+            }
+            continue;
         }
         const long long lo = W * b / G, hi = W * (b + 1) / G;
         while (idx < N && pos + t3[idx].w <= lo) pos += t3[idx++].w;
@@ -551,6 +585,7 @@ int BuildLists(ptk_batch *B) {
     B->hCounts[8] = (int)B->gbTiles.n;
     B->hCounts[9] = (int)B->gbHalves.n;
     B->hCounts[10] = (int)B->gbQuarters.n;
+    B->hCounts[11] = three && t3.size() < (size_t)B->grid3;  // BatchFdtdSteps3's tile body
     auto up = [&](auto &l) -> int {
         if (l.n) HIPCHK(ptk_hip_memcpy_htod_async(l.dev, l.host, l.n * sizeof(*l.host), B->stream));
         return PTK_BATCH_OK;

@@ -102,20 +102,21 @@ BatchFdtdStep(const int4 *__restrict__ tiles, const int *__restrict__ count, con
     }
 }
 
-// Three whole Yee steps per launch on overlapped tiles (overlapn_tile<3>, fdtd_fused.h) over a
-// persistent schedule of G virtual blocks (count[1]): virtual block b's items are
-// [starts[b], starts[b+1]) of `tiles`, each {inst, tile x, tile y, k0 | k1 << 16} of 58 x 10
-// owned columns, taken in order.  The executor builds the schedule (whole-depth tiles round-robin,
-// then equal runs of the remaining tiles' planes); blocks of 64 x 16 threads take virtual blocks
-// in grid strides, XCD-contiguously, so any grid size covers every item once.  A launch reads
-// set (done & 1) and writes the other set three steps later, so one BatchFdtdAdvance per launch
-// keeps the set index right.  Same instance conditions as BatchFdtdStep.
-extern "C" __global__ void __launch_bounds__(1024)
-BatchFdtdSteps3(const int4 *__restrict__ tiles, const int *__restrict__ count, const int *__restrict__ starts,
-                const PTK_FDTD_INST *__restrict__ insts) {
-    __shared__ OverlapNLds<3, 16, 1> L;
-    if (blockDim.x != 64 || blockDim.y != 16 || blockDim.z != 1) return;  // geometry contract
-    const int G = count[1];
+// Three whole Yee steps per launch on overlapped tiles over a persistent schedule of G virtual
+// blocks (count[1]): virtual block b's items are [starts[b], starts[b+1]) of `tiles`, each {inst,
+// tile x, tile y, k0 | k1 << 16} of 58 x 10 owned columns, taken in order.  The executor builds the
+// schedule (whole-depth tiles round-robin, then segments of the remaining tiles); blocks of 64 x 16
+// threads take virtual blocks in grid strides, XCD-contiguously, so any grid size covers every item
+// once.  A launch reads set (done & 1) and writes the other set three steps later, so one
+// BatchFdtdAdvance per launch keeps the set index right.  Same instance conditions as BatchFdtdStep.
+// count[5]: there are fewer tiles than virtual blocks.  Then a launch lasts as long as one segment's
+// planes, and column_tile forms them (fdtd_fused.h): 24 instances of edge 16..40, 29 us per launch
+// against 50 with overlapn_tile on equal runs.  With more tiles (2048 instances of edge 16..96)
+// HBM and the overlap's reuse in L2 count, as at 384^3, and overlapn_tile is the faster: 205 ms of
+// execution for 50 steps against 215.
+template <class Tile>
+__device__ __forceinline__ void batch_steps3(const int4 *__restrict__ tiles, int G, const int *__restrict__ starts,
+                                             const PTK_FDTD_INST *__restrict__ insts, Tile tile) {
     for (int vb = (int)blockIdx.x; vb < G; vb += (int)gridDim.x) {
         const int b = (int)gb_xcd_block((unsigned)vb, (unsigned)G);
         for (int t = starts[b]; t < starts[b + 1]; ++t) {
@@ -126,10 +127,27 @@ BatchFdtdSteps3(const int4 *__restrict__ tiles, const int *__restrict__ count, c
             const Fields F{I.f[cur][0], I.f[cur][1], I.f[cur][2], I.f[cur][3], I.f[cur][4], I.f[cur][5],
                            I.f[nxt][0], I.f[nxt][1], I.f[nxt][2], I.f[nxt][3], I.f[nxt][4], I.f[nxt][5]};
             const int k0 = tl.w & 0xffff, k1 = (int)((unsigned)tl.w >> 16);
-            overlapn_tile<3, 16>(F, I.p, tl.y * 58, tl.z * 10, k0, k1, L);
+            tile(F, I.p, tl.y * 58, tl.z * 10, k0, k1);
             lds_barrier();  // the next item reuses LDS
         }
     }
+}
+
+extern "C" __global__ void __launch_bounds__(1024)
+BatchFdtdSteps3(const int4 *__restrict__ tiles, const int *__restrict__ count, const int *__restrict__ starts,
+                const PTK_FDTD_INST *__restrict__ insts) {
+    __shared__ union {
+        OverlapNLds<3, 16, 1> o;
+        ColumnLds<3, 16> c;
+    } L;
+    if (blockDim.x != 64 || blockDim.y != 16 || blockDim.z != 1) return;  // geometry contract
+    const int G = count[1];
+    if (count[5])
+        batch_steps3(tiles, G, starts, insts, [&](const Fields &F, const FDTD_PARAMS &p, int i0, int j0, int k0, int k1)
+                     __attribute__((always_inline)) { column_tile<3, 16>(F, p, i0, j0, k0, k1, L.c); });
+    else
+        batch_steps3(tiles, G, starts, insts, [&](const Fields &F, const FDTD_PARAMS &p, int i0, int j0, int k0, int k1)
+                     __attribute__((always_inline)) { overlapn_tile<3, 16>(F, p, i0, j0, k0, k1, L.o); });
 }
 
 extern "C" __global__ void __launch_bounds__(256)

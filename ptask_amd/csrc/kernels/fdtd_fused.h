@@ -21,6 +21,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ptk_fdtd.h"
 
 namespace ptk_fdtd {
@@ -233,6 +235,10 @@ __device__ inline void lds_barrier() {
 // Lane 63 reads 0; it is a halo lane of every tile.
 __device__ inline float lane_next(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xF, 0xF, false));
+}
+
+__device__ inline float lane_prev(float v) {  // lane l reads lane l - 1 (wave_shr:1), lane 0 reads 0
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xF, 0xF, false));
 }
 
 // Raw buffer access to one field array.  A byte offset at or beyond the array's size reads 0
@@ -603,6 +609,232 @@ __device__ inline void overlapn_tile(const Fields &F, const FDTD_PARAMS &p, int 
         plane(m + 2, S2, S3, S1);
         plane(m + 3, S3, S0, S2);
     }
+}
+
+// ---- the same tiles with every lane's column in registers ------------------------------------------
+//
+// column_tile computes what overlapn_tile computes, over the same tiles and with the same pipeline
+// of steps, with less work per plane for problems whose time is a plane's latency rather than HBM:
+// a lane keeps its own column of every step in registers (of each step the two planes that step s + 1
+// still needs, in two slots by iteration parity; within an iteration the steps go from T down to 1, so
+// a slot is overwritten just after its last use and nothing is copied), i - 1 and i + 1 are the
+// neighbouring lanes (a DPP operand), and only the row neighbours cross waves, through LDS planes by
+// iteration parity: Ex and Ez of row j + 1 for A, Hx and Hz of row j - 1 for B.
+//   h[s]  written in A of iteration m, read in B of m, written again in A of m + 2;
+//   e[s]  written in B of m (the inputs' in A of m - 1), read in A of m + 2 (m), written again in B
+//         of m + 2 (A of m + 1): each pair has a barrier between, so the one barrier between A and
+//         B orders every access.
+// A step is formed only in the iterations that need it: with T = 3, owned planes [k0, k1) need H_s
+// from iteration 3(s - 1) on (counted from plane k0 - T) and E_s up to T - s iterations before the
+// last, so a slab of n planes takes n + 7 iterations and 3n + 9 step planes instead of 3n + 21: most
+// of the work of the short slabs that a small problem is cut into.
+// Measured: 64^3, three steps on 256 blocks: 22.0 us per launch against 41.9 (35.5 before the short
+// slabs and the skipped steps, 25.1 with the slabs alone).  At 384^3
+// it is the slower one, 890 us against 755: it computes a launch in 460 us when nothing is read or
+// written, so the blocks run at the pace of memory and drift apart, and neighbouring tiles then fetch
+// the three cells they share twice (FETCH_SIZE 2.12 GB against 1.67).  overlapn_tile's two barriers
+// and fuller planes keep the blocks in step.  So this body serves the launches with fewer tiles than
+// blocks (and the batched small instances), overlapn_tile the others.
+template <int T, int MAXR>
+struct ColumnLds {
+    float e[T][2][2][MAXR + 1][64]; // Ex, Ez of E_0 .. E_{T-1}: row r's at [r]
+    float h[T][2][2][MAXR + 1][64]; // Hx, Hz of H_1 .. H_T: row r's at [r + 1]
+};
+
+// A field of `bytes` bytes from the row at byte offset `row` of its first plane on; a plane is then
+// addressed by its byte offset in a scalar register and a 32-bit lane part.  Loads are clamped into
+// the field (what is read outside it reaches no stored cell).  A lane that stores nothing carries
+// bit 31 in its part, which the buffer unit's range check drops whether or not it counts the scalar
+// part (their sum stays below 2^32); the scalar part is that of a plane inside the field.
+__device__ inline PlaneBuf row_buf(const float *p, unsigned bytes, unsigned row) {
+    return plane_buf((const float *)((const char *)p + row), bytes - row);
+}
+
+// A value that is the same in every lane, in a scalar register.
+__device__ inline unsigned uni(unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); }
+
+template <int T, int MAXR>
+__device__ inline void column_tile(const Fields &F, const FDTD_PARAMS &p, int i0, int j0, int k0, int k1,
+                                   ColumnLds<T, MAXR> &L) {
+    static_assert(T == 3, "the iterations below are those of three steps");
+    const Coef c = make_coef(p);
+    i0 = (int)uni((unsigned)i0), j0 = (int)uni((unsigned)j0), k0 = (int)uni((unsigned)k0), k1 = (int)uni((unsigned)k1);
+    const int R = (int)blockDim.y;
+    const int l = (int)threadIdx.x, r = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int i = i0 - T + l, j = j0 - T + r;
+    const int Nx = p.Nx, Ny = p.Ny, Nz = p.Nz;
+    auto clamp = [](int v, int hi) { return v < 0 ? 0 : v < hi ? v : hi; };
+    // lane offsets of the fields with Nx + 1 and with Nx cells per row; bit 31 where nothing is stored
+    const unsigned c1 = 4u * (unsigned)clamp(i, Nx), c0 = 4u * (unsigned)clamp(i, Nx - 1);
+    const bool ownL = l >= T && l <= 63 - T, ownR = r >= T && r <= R - 1 - T;
+    const unsigned n1 = uni(ownR && j <= Ny ? 0u : kNoCell), n0 = uni(ownR && j < Ny ? 0u : kNoCell);
+    // lane parts of the stores to the four extents (see below)
+    const unsigned l1 = ownL && i <= Nx ? c1 : kNoCell, l0 = ownL && i < Nx ? c0 : kNoCell;
+    const unsigned lA = l1 | n0, lB = l0 | n1, lC = l0 | n0, lD = l1 | n1;
+    // row offsets and plane strides of the four extents: (Nx+1, Ny) Hx Ey, (Nx, Ny+1) Hy Ex, (Nx, Ny) Hz,
+    // (Nx+1, Ny+1) Ez
+    const int j1 = clamp(j, Ny), j0r = clamp(j, Ny - 1);
+    const unsigned rA = uni(4u * (Nx + 1) * j0r), rB = uni(4u * Nx * j1), rC = uni(4u * Nx * j0r), rD = uni(4u * (Nx + 1) * j1);
+    const unsigned sA = 4u * (Nx + 1) * Ny, sB = 4u * Nx * (Ny + 1), sC = 4u * Nx * Ny, sD = 4u * (Nx + 1) * (Ny + 1);
+    const PlaneBuf rHx = row_buf(F.hx, sA * Nz, rA), rHy = row_buf(F.hy, sB * Nz, rB), rHz = row_buf(F.hz, sC * (Nz + 1), rC),
+                   rEx = row_buf(F.ex, sB * (Nz + 1), rB), rEy = row_buf(F.ey, sA * (Nz + 1), rA), rEz = row_buf(F.ez, sD * Nz, rD);
+    const PlaneBuf wHx = row_buf(F.ohx, sA * Nz, rA), wHy = row_buf(F.ohy, sB * Nz, rB), wHz = row_buf(F.ohz, sC * (Nz + 1), rC),
+                   wEx = row_buf(F.oex, sB * (Nz + 1), rB), wEy = row_buf(F.oey, sA * (Nz + 1), rA), wEz = row_buf(F.oez, sD * Nz, rD);
+    const bool jIn = j >= 1 && j <= Ny - 1, iIn = i >= 1 && i <= Nx - 1;
+
+    struct Set {
+        F3 e, h;
+    };
+    // S_m = {E_0(m+1), H_0(m)}.  The owned planes below k1 depend on input planes up to T above
+    // them (each step reaches one plane up), so only m <= k1 + T - 2 feed owned cells; a later
+    // set reloads that set's planes (cached) and a plane outside a field is read as its first or
+    // last: those values reach no stored cell, as the planes formed from them do not (E of plane 0
+    // and of plane Nz is copied through, whatever the planes beyond).
+    auto load_set = [&](Set &S, int m) {
+        const int k = m < k1 + T - 2 ? m : k1 + T - 2;
+        const unsigned ke = clamp(k + 1, Nz), kez = clamp(k + 1, Nz - 1), kh = clamp(k, Nz - 1), khz = clamp(k, Nz);
+        S.e.x = rEx.load(c0, ke * sB);
+        S.e.y = rEy.load(c1, ke * sA);
+        S.e.z = rEz.load(c1, kez * sD);
+        S.h.x = rHx.load(c1, kh * sA);
+        S.h.y = rHy.load(c0, kh * sB);
+        S.h.z = rHz.load(c0, khz * sC);
+    };
+    // six dropped stores: the prologue then leaves the memory counter as a loop iteration does,
+    // so the waits the compiler places in the loop stay two planes behind the loads
+    auto pad_stores = [&]() {
+        wHx.store(kNoCell, 0u, 0.f);
+        wHy.store(kNoCell, 0u, 0.f);
+        wHz.store(kNoCell, 0u, 0.f);
+        wEx.store(kNoCell, 0u, 0.f);
+        wEy.store(kNoCell, 0u, 0.f);
+        wEz.store(kNoCell, 0u, 0.f);
+    };
+    constexpr int kLag = 2 * (T - 1);
+    const int ms = k0 - T;  // the first iteration's plane (see above); the last is k1 - 1 + kLag
+    Set S0, S1, S2, S3;
+    {
+        const unsigned ke = clamp(ms, Nz), kez = clamp(ms, Nz - 1);
+        S0.e.x = rEx.load(c0, ke * sB);  // E_0(ms)
+        S0.e.y = rEy.load(c1, ke * sA);
+        S0.e.z = rEz.load(c1, kez * sD);
+        S0.h = F3{0.f, 0.f, 0.f};
+    }
+    load_set(S1, ms);
+    pad_stores();
+    load_set(S2, ms + 1);
+    pad_stores();
+    // this lane's row of an LDS plane; the other planes and rows are constant offsets from it (the
+    // empty asm keeps the two bases in registers instead of a sum per access)
+    typedef __attribute__((address_space(3))) float Lds;
+    Lds *eb = (Lds *)&L.e[0][0][0][r][l], *hb = (Lds *)&L.h[0][0][0][r][l];
+    asm("" : "+v"(eb), "+v"(hb));
+    constexpr int kRow = 64, kPlane = (MAXR + 1) * kRow;
+    auto ls = [](Lds *q, int s, int par, int comp, int row) -> Lds & { return q[((s * 2 + par) * 2 + comp) * kPlane + row * kRow]; };
+    ls(eb, 0, 0, 0, 0) = S0.e.x;  // iteration ms has parity 0
+    ls(eb, 0, 0, 1, 0) = S0.e.z;
+    // own columns of steps 1 .. T by iteration parity (index 0 unused)
+    F3 E[T + 1][2], H[T + 1][2];
+#pragma unroll
+    for (int s = 0; s <= T; ++s) E[s][0] = E[s][1] = H[s][0] = H[s][1] = F3{0.f, 0.f, 0.f};
+
+    lds_barrier();
+    // iteration m, forming steps lo .. hi; P, S, N: sets m - 1, m, m + 2
+    auto plane = [&](int m, auto parity, auto lo_, auto hi_, const Set &P, const Set &S, Set &N) {
+        constexpr int b = decltype(parity)::value, lo = decltype(lo_)::value, hi = decltype(hi_)::value;
+        if (lo == 1) {
+            load_set(N, m + 2);
+            // issue the loads of the plane two ahead before this plane's LDS traffic and its waits
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // ---- A: H_s(p_s) for every step
+        float xj[T], zj[T];  // Ex, Ez of E_{s-1}(p_s) in row j + 1: read before anything is written
+#pragma unroll
+        for (int s = hi; s >= lo; --s) {
+            xj[s - 1] = ls(eb, s - 1, b, 0, 1);
+            zj[s - 1] = ls(eb, s - 1, b, 1, 1);
+        }
+#pragma unroll
+        for (int s = hi; s >= lo; --s) {
+            const F3 ep = s == 1 ? P.e : E[s - 1][b], eu = s == 1 ? S.e : E[s - 1][b ^ 1];
+            const F3 ho = s == 1 ? S.h : H[s - 1][b];
+            const float exj = xj[s - 1], ezj = zj[s - 1];
+            F3 &hn = H[s][b];
+            hn.x = ho.x + c.cH * ((eu.y - ep.y) * c.Cz - (ezj - ep.z) * c.Cy);
+            hn.y = ho.y + c.cH * ((lane_next(ep.z) - ep.z) * c.Cx - (eu.x - ep.x) * c.Cz);
+            hn.z = ho.z + c.cH * ((exj - ep.x) * c.Cy - (lane_next(ep.y) - ep.y) * c.Cx);
+            ls(hb, s - 1, b, 0, 1) = hn.x;
+            ls(hb, s - 1, b, 1, 1) = hn.z;
+        }
+        if (lo == 1) {
+            ls(eb, 0, b ^ 1, 0, 0) = S.e.x;
+            ls(eb, 0, b ^ 1, 1, 0) = S.e.z;
+        }
+        lds_barrier();
+        // ---- B: E_s(p_s) for every step (graphfdtd.cpp:243-312: interior cells update, faces
+        // copy through)
+        F3 out;
+#pragma unroll
+        for (int s = hi; s >= lo; --s) {  // Hx, Hz of H_s(p_s) in row j - 1
+            xj[s - 1] = ls(hb, s - 1, b, 0, 0);
+            zj[s - 1] = ls(hb, s - 1, b, 1, 0);
+        }
+#pragma unroll
+        for (int s = hi; s >= lo; --s) {
+            const int ps = m - 2 * (s - 1);
+            const bool kIn = ps >= 1 && ps <= Nz - 1;
+            const F3 e = s == 1 ? P.e : E[s - 1][b];
+            const F3 hn = H[s][b], hp = H[s][b ^ 1];
+            const float hxj = xj[s - 1], hzj = zj[s - 1];
+            const float wx = e.x + c.cE * ((hn.z - hzj) * c.Cy - (hn.y - hp.y) * c.Cz);
+            const float wy = e.y + c.cE * ((hn.x - hp.x) * c.Cz - (hn.z - lane_prev(hn.z)) * c.Cx);
+            const float wz = e.z + c.cE * ((hn.y - lane_prev(hn.y)) * c.Cx - (hn.x - hxj) * c.Cy);
+            F3 &en = s == T ? out : E[s][b];
+            en.x = (jIn && kIn) ? wx : e.x;
+            en.y = (iIn && kIn) ? wy : e.y;
+            en.z = (iIn && jIn) ? wz : e.z;
+            if (s < T) {
+                ls(eb, s, b, 0, 0) = en.x;
+                ls(eb, s, b, 1, 0) = en.z;
+            }
+        }
+        if (hi < T) {
+            pad_stores();
+            return;
+        }
+        // plane q of each output if it is in the slab and the field
+        const int q = m - kLag;
+        const bool in = q >= k0 && q < k1;
+        const unsigned q0 = uni(in && q < Nz ? 0u : kNoCell), q1 = uni(in ? 0u : kNoCell);
+        const unsigned k1q = (unsigned)clamp(q, Nz), k0q = (unsigned)clamp(q, Nz - 1);
+        wHx.store(lA | q0, k0q * sA, H[T][b].x);
+        wHy.store(lB | q0, k0q * sB, H[T][b].y);
+        wHz.store(lC | q1, k1q * sC, H[T][b].z);
+        wEx.store(lB | q1, k1q * sB, out.x);
+        wEy.store(lA | q1, k1q * sA, out.y);
+        wEz.store(lD | q0, k0q * sD, out.z);
+    };
+    // The sets rotate through four iterations.  The loop runs whole groups of four with no branch
+    // inside: up to three planes past the slab are formed and discarded (q >= k1: nothing stored).
+    typedef std::integral_constant<int, 0> Even;
+    typedef std::integral_constant<int, 1> Odd, One;
+    typedef std::integral_constant<int, 2> Two;
+    typedef std::integral_constant<int, 3> Three;
+    int m = ms;
+    plane(m, Even{}, One{}, One{}, S0, S1, S3);
+    plane(m + 1, Odd{}, One{}, One{}, S1, S2, S0);
+    plane(m + 2, Even{}, One{}, One{}, S2, S3, S1);
+    plane(m + 3, Odd{}, One{}, Two{}, S3, S0, S2);
+    plane(m + 4, Even{}, One{}, Two{}, S0, S1, S3);
+    plane(m + 5, Odd{}, One{}, Two{}, S1, S2, S0);
+    for (m += 6; m < k1 + 2; m += 4) {  // iterations 6 .. n + 4
+        plane(m, Even{}, One{}, Three{}, S2, S3, S1);
+        plane(m + 1, Odd{}, One{}, Three{}, S3, S0, S2);
+        plane(m + 2, Even{}, One{}, Three{}, S0, S1, S3);
+        plane(m + 3, Odd{}, One{}, Three{}, S1, S2, S0);
+    }
+    plane(m, Even{}, Two{}, Three{}, S2, S3, S1);
+    plane(m + 1, Odd{}, Three{}, Three{}, S3, S0, S2);
 }
 
 }  // namespace ptk_fdtd

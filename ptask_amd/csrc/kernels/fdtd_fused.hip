@@ -138,12 +138,23 @@ OVERLAPN_KERNEL(FdtdThreeStepOverlap, 3, 1)
 // The same T steps with a persistent 1-D grid of G blocks (one per CU): the N tiles split into
 // q = N / G whole-depth tiles per block, taken by all blocks together from plane 0 upwards (the
 // tiles live at the same time share their i/j overlap in L2), and the planes of the remaining
-// N - qG tiles cut into G equal runs in (tile, plane) order, one per block.  Every block then
-// streams q(Nz+1) + (N - qG)(Nz+1)/G planes plus the pipeline's lag once or twice, instead of
-// whole slabs in rounds of G blocks.  Any G covers every tile and plane exactly once.  Launch:
-// block (64, R, 1), grid (G, 1, 1).
-template <int T, int HB>
-__device__ inline void overlapn_persistent(const Fields &F, const FDTD_PARAMS &p, OverlapNLds<T, 16, HB> &L) {
+// M = N - qG tiles cut among the G blocks.  A segment of n planes costs n plus the pipeline's T + 2(T-1)
+// planes, so the cut is one of two: each tile into G / M equal slabs (or one more), one per block, or,
+// when that leaves too many blocks idle (M just below G), G equal runs in (tile, plane) order, most
+// of which cross from one tile into the next and pay the pipeline twice.  At 64^3 (14 tiles on 256
+// blocks) slabs of 4 planes take 12 plane iterations per block, runs of 3.6 up to 24.
+// Any G covers every tile and plane exactly once.  Launch: block (64, R, 1), grid (G, 1, 1).
+// With fewer tiles than blocks the planes' latency is what counts: column_tile; see there.
+template <int T>
+struct PersistentLds {
+    union {
+        OverlapNLds<T, 16, 1> o;
+        ColumnLds<T, 16> c;
+    };
+};
+
+template <int T>
+__device__ inline void overlapn_persistent(const Fields &F, const FDTD_PARAMS &p, PersistentLds<T> &L) {
     const int R = (int)blockDim.y;
     if (blockDim.x != 64 || R < 2 * T + 1 || R > 16 || blockDim.z != 1) return;  // geometry contract
     if (gridDim.y != 1 || gridDim.z != 1) return;
@@ -156,10 +167,29 @@ __device__ inline void overlapn_persistent(const Fields &F, const FDTD_PARAMS &p
         const int xcd = b % kNumXcd, local = b / kNumXcd, per = G / kNumXcd, rem = G % kNumXcd;
         b = xcd * per + (xcd < rem ? xcd : rem) + local;
     }
-    const int q = N / G;
-    const long long W = (long long)(N - q * G) * D;  // tile-planes left after the whole tiles
-    long long w = W * b / G;
-    const long long hi = W * (b + 1) / G;
+    const int q = N / G, M = N - q * G;  // M < G
+    constexpr int kPipe = T + 2 * (T - 1);
+    const bool slabs = M > 0 && (D + G / M - 1) / (G / M) + kPipe <= (int)((long long)M * D / G) + 2 * kPipe;
+    long long w, hi;  // this block's run of the remaining tiles' planes
+    if (slabs) {      // block b is one of the blocks [f0, f1) of tile b M / G
+        const int t = (int)((long long)b * M / G);
+        const int f0 = (int)(((long long)t * G + M - 1) / M), f1 = (int)(((long long)(t + 1) * G + M - 1) / M);
+        w = (long long)t * D + (long long)D * (b - f0) / (f1 - f0);
+        hi = (long long)t * D + (long long)D * (b - f0 + 1) / (f1 - f0);
+    } else {
+        const long long W = (long long)M * D;
+        w = W * b / G;
+        hi = W * (b + 1) / G;
+    }
+    if (q == 0) {
+        while (w < hi) {  // a run of the tiles' planes, a tile at a time
+            const int t = (int)(w / D), k0 = (int)(w % D), k1 = (int)(k0 + (hi - w) < D ? k0 + (hi - w) : D);
+            column_tile<T, 16>(F, p, (t % ti) * ow, (t / ti) * oh, k0, k1, L.c);
+            w += k1 - k0;
+            lds_barrier();  // the next segment reuses LDS
+        }
+        return;
+    }
     // one call site for both kinds of segment (the tile body is large)
     for (int r = 0;; ++r) {
         int t, k0, k1;
@@ -172,7 +202,7 @@ __device__ inline void overlapn_persistent(const Fields &F, const FDTD_PARAMS &p
         } else {
             break;
         }
-        overlapn_tile<T, 16>(F, p, (t % ti) * ow, (t / ti) * oh, k0, k1, L);
+        overlapn_tile<T, 16>(F, p, (t % ti) * ow, (t / ti) * oh, k0, k1, L.o);
         lds_barrier();  // the next segment reuses LDS
     }
 }
@@ -181,9 +211,9 @@ extern "C" __global__ void __launch_bounds__(1024)
 FdtdThreeStepPersistent(const float *hx, const float *hy, const float *hz, const float *ex, const float *ey,
                         const float *ez, FDTD_PARAMS p, float *ohx, float *ohy, float *ohz, float *oex,
                         float *oey, float *oez) {
-    __shared__ OverlapNLds<3, 16, 1> L;
+    __shared__ PersistentLds<3> L;
     const Fields F{hx, hy, hz, ex, ey, ez, ohx, ohy, ohz, oex, oey, oez};
-    overlapn_persistent<3, 1>(F, p, L);
+    overlapn_persistent<3>(F, p, L);
 }
 
 // ---- half-step kernels: all three H updates in one streaming pass, then all three E updates ----
