@@ -21,6 +21,8 @@
 // length-M vectors are binary64.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ptk_pca.h"
 
 // Tolerance-checked binary32 work: let the compiler fuse multiply-adds (the build default is off).
@@ -274,8 +276,8 @@ PcaDeflate(float *__restrict__ R, float *__restrict__ T, float *__restrict__ S, 
 
 // ---- PcaReduce: red[g][n] = sum of part[b][n] over the g-th of GR contiguous groups of the G
 // rows.  Grid (ceil(ld/64), GR) blocks of 256 (64 columns x 4 interleaved row subsets).  The
-// loads read clamped, always valid rows unconditionally, eight at a time, so they issue together;
-// the sums take the valid terms in row order.
+// loads read clamped, always valid rows unconditionally, sixteen at a time, so they issue together
+// (384 rows in 8 groups are 12 per thread: one round trip); the sums take the valid terms in row order.
 extern "C" __global__ void __launch_bounds__(256)
 PcaReduce(float *__restrict__ S, PCA_DIMS d) {
     __shared__ double sh[4][64];
@@ -285,15 +287,15 @@ PcaReduce(float *__restrict__ S, PCA_DIMS d) {
     const int lo = (int)((long long)g * d.G / d.GR), hi = (int)((long long)(g + 1) * d.G / d.GR);
     const float *part = pca_part(S, d);
     double s = 0;
-    for (int b0 = lo + sub; b0 < hi; b0 += 32) {
-        float x[8];
+    for (int b0 = lo + sub; b0 < hi; b0 += 64) {
+        float x[16];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < 16; ++u) {
             const int b = b0 + 4 * u < hi ? b0 + 4 * u : hi - 1;
             x[u] = part[(long long)b * ld + cc];
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+        for (int u = 0; u < 16; ++u)
             if (b0 + 4 * u < hi) s += (double)x[u];
     }
     sh[sub][c] = col < ld ? s : 0.0;
@@ -303,120 +305,185 @@ PcaReduce(float *__restrict__ S, PCA_DIMS d) {
 
 // ---- PcaOrthonormalize: one block of 1024.  p = sum of the GR rows of red; classical
 // Gram-Schmidt against the components before k (U = P_<k^T p, then p -= P_<k U: pca_cpu.cpp:356-372);
-// p *= 1/|p| (dnrm2 + dscal: pca_cpu.cpp:374-376); P[k] = p.  EPT elements per thread (ld <=
-// 1024 * EPT).  Loads read clamped, always valid addresses unconditionally, in groups of eight
-// rows, so a group's loads issue together; each sum then takes its valid terms in order.
+// p *= 1/|p| (dnrm2 + dscal: pca_cpu.cpp:374-376); P[k] = p.
+//
+// One block, so its time is a chain of latencies and what one CU can load and exchange, and the
+// kernel is built to keep that chain short: a thread owns EPT consecutive columns, the loads of the
+// first CH rows of P are issued together with those of red and stay in registers for both uses, and
+// the dot products are reduced by halving (below), not each on its own.  Average over k = 0 .. 15
+// at 2048 columns: 7.2 us, and 5.3 us over k = 0 .. 3 at 700 columns; 12.0 and 8.4 us with a shuffle
+// tree per dot product (2 x 6 x k LDS exchanges in each of the 16 waves) and the rows of P loaded
+// again for the second use.
+
+// 16 lanes of a DPP row: a value from the lane that mirrors this one in its row, its half row, its
+// quad, and its pair.
+template <int CTRL>
+__device__ __forceinline__ double pca_dpp(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+constexpr int kRowMirror = 0x140, kHalfMirror = 0x141, kQuadMirror = 0x1B, kPairSwap = 0xB1;
+
+// Sum of v over the 16 lanes of the row, in every lane.
+__device__ __forceinline__ double pca_row_sum(double v) {
+    v += pca_dpp<kRowMirror>(v);
+    v += pca_dpp<kHalfMirror>(v);
+    v += pca_dpp<kQuadMirror>(v);
+    return v + pca_dpp<kPairSwap>(v);
+}
+
+// Sixteen sums over the row's lanes at once: lane l of the row gets the sum of v[l & 15].  At each step
+// a lane gives its partner the half of the sums that the partner keeps: 15 exchanges and additions
+// for all sixteen instead of 64.
+__device__ __forceinline__ double pca_row_sum16(double (&v)[16], int l16) {
+    auto step = [&](auto ctrl, int n, bool up) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (i < n) {
+                const double give = up ? v[i] : v[i + n], keep = up ? v[i + n] : v[i];
+                v[i] = keep + pca_dpp<decltype(ctrl)::value>(give);
+            }
+    };
+    step(std::integral_constant<int, kRowMirror>{}, 8, (l16 & 8) != 0);
+    step(std::integral_constant<int, kHalfMirror>{}, 4, (l16 & 4) != 0);
+    step(std::integral_constant<int, kQuadMirror>{}, 2, (l16 & 2) != 0);
+    step(std::integral_constant<int, kPairSwap>{}, 1, (l16 & 1) != 0);
+    return v[0];
+}
+
+struct PcaOrthoLds {
+    double w[64][PTK_PCA_MAX_K + 1];  // per DPP row of the block: its part of the dot products (rows
+                                      // of an odd number of doubles: a column's parts spread over the banks)
+    double u[PTK_PCA_MAX_K];
+    double n[64];
+};
+
+// A load of E consecutive elements (E = 1, 2 or 4; aligned to as many).
+template <int E, class T>
+__device__ __forceinline__ void pca_load(const T *__restrict__ p, T (&v)[E]) {
+    typedef T V __attribute__((ext_vector_type(E)));
+    const V x = *(const V *)p;
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = x[e];
+}
+template <>
+__device__ __forceinline__ void pca_load<1, float>(const float *__restrict__ p, float (&v)[1]) { v[0] = *p; }
+template <>
+__device__ __forceinline__ void pca_load<1, double>(const double *__restrict__ p, double (&v)[1]) { v[0] = *p; }
+
 template <int EPT>
-__device__ inline void pca_orthonormalize(float *__restrict__ S, const PCA_DIMS &d, double (&sW)[16][PTK_PCA_MAX_K],
-                                          double (&sU)[PTK_PCA_MAX_K]) {
-    constexpr int kGroup = 8;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, ld = d.ld, k = d.k, GR = d.GR;
-    const double *red = pca_red(S, d);
+__device__ inline void pca_orthonormalize(float *__restrict__ S, const PCA_DIMS &d, PcaOrthoLds &L) {
+    constexpr int CH = 16;               // rows of P reduced together
+    constexpr int RG = EPT == 4 ? 4 : 8; // rows of red loaded together
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, row = tid >> 4, ld = d.ld, k = d.k, GR = d.GR;
+    const double *__restrict__ red = pca_red(S, d);
     float *P = pca_P(S, d);
-    int nc[EPT];
-    bool nv[EPT];
+    // columns n0 .. n0 + EPT - 1: ld is a multiple of 4, so all of them or none are in range; a
+    // thread past the end reads the last ones and adds nothing
+    const bool on = tid * EPT < ld;
+    const int n0 = on ? tid * EPT : ld - EPT;
+    // rows [j0, j0 + CH) of P below k, four at a time as far as they reach; the others as zeros
+    float pv[CH][EPT];
+    auto loadP = [&](int j0) {
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-        const int n = tid + 1024 * i;
-        nv[i] = n < ld;
-        nc[i] = n < ld ? n : ld - 1;
-    }
-    double p[EPT];
+        for (int q = 0; q < CH; q += 4) {
+            if (j0 + q < k) {
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) p[i] = 0;
-    for (int g0 = 0; g0 < GR; g0 += kGroup) {
-        double rv[kGroup][EPT];
+                for (int i = q; i < q + 4; ++i) pca_load<EPT>(P + (long long)(j0 + i < k ? j0 + i : k - 1) * ld + n0, pv[i]);
+            } else {
 #pragma unroll
-        for (int gg = 0; gg < kGroup; ++gg) {
-            const int g = g0 + gg < GR ? g0 + gg : GR - 1;
+                for (int i = q; i < q + 4; ++i)
 #pragma unroll
-            for (int i = 0; i < EPT; ++i) rv[gg][i] = red[(long long)g * ld + nc[i]];
-        }
-#pragma unroll
-        for (int gg = 0; gg < kGroup; ++gg)
-            if (g0 + gg < GR)
-#pragma unroll
-                for (int i = 0; i < EPT; ++i)
-                    if (nv[i]) p[i] += rv[gg][i];
-    }
-    auto loadP = [&](float (&pv)[kGroup][EPT], int j0) {
-#pragma unroll
-        for (int jj = 0; jj < kGroup; ++jj) {
-            const int j = j0 + jj < k ? j0 + jj : k - 1;
-#pragma unroll
-            for (int i = 0; i < EPT; ++i) pv[jj][i] = P[(long long)j * ld + nc[i]];
+                    for (int e = 0; e < EPT; ++e) pv[i][e] = 0.f;
+            }
         }
     };
+    loadP(0);
+    double p[EPT];
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) p[e] = 0;
+    for (int g0 = 0; g0 < GR; g0 += RG) {
+        double rv[RG][EPT];
+#pragma unroll
+        for (int g = 0; g < RG; ++g) pca_load<EPT>(red + (long long)(g0 + g < GR ? g0 + g : GR - 1) * ld + n0, rv[g]);
+#pragma unroll
+        for (int g = 0; g < RG; ++g)
+            if (g0 + g < GR)
+#pragma unroll
+                for (int e = 0; e < EPT; ++e) p[e] += rv[g][e];
+    }
+    if (!on)
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) p[e] = 0;
     if (k > 0) {
-        // the k dot products eight at a time; the eight wave reductions run together
-        for (int j0 = 0; j0 < k; j0 += kGroup) {
-            float pv[kGroup][EPT];
-            loadP(pv, j0);
-            double v[kGroup];
+        for (int j0 = 0; j0 < k; j0 += CH) {
+            if (j0 > 0) loadP(j0);
+            double v[CH];
 #pragma unroll
-            for (int jj = 0; jj < kGroup; ++jj) {
-                v[jj] = 0;
-                if (j0 + jj < k)
+            for (int i = 0; i < CH; ++i) {
+                v[i] = (double)pv[i][0] * p[0];  // a row past k - 1 may repeat it; its sum is not used
 #pragma unroll
-                    for (int i = 0; i < EPT; ++i)
-                        if (nv[i]) v[jj] += (double)pv[jj][i] * p[i];
+                for (int e = 1; e < EPT; ++e) v[i] = fma((double)pv[i][e], p[e], v[i]);
             }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-                for (int jj = 0; jj < kGroup; ++jj) v[jj] += __shfl_xor(v[jj], off, 64);
-            if (lane == 0)
-#pragma unroll
-                for (int jj = 0; jj < kGroup; ++jj)
-                    if (j0 + jj < k) sW[wv][j0 + jj] = v[jj];
+            const double t = pca_row_sum16(v, l16);
+            L.w[row][j0 + l16] = t;
         }
         __syncthreads();
-        if (tid < k) {
+        {   // U_j: sixteen threads a component, each four of the 64 rows' parts in order, then the row sum
+            const int j = tid >> 4;  // 64 components
             double u = 0;
-            for (int w = 0; w < 16; ++w) u += sW[w][tid];
-            sU[tid] = u;
+            if (j < k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) u += L.w[4 * l16 + i][j];
+            u = pca_row_sum(u);
+            if (l16 == 0) L.u[j] = j < k ? u : 0.0;
         }
         __syncthreads();
-        // p -= P_<k U: each element's sum over j in order
+        // p -= P_<k U: each element's sum over j in order.  Only more than CH rows are loaded again.
         double s[EPT];
 #pragma unroll
-        for (int i = 0; i < EPT; ++i) s[i] = 0;
-        for (int j0 = 0; j0 < k; j0 += kGroup) {
-            float pv[kGroup][EPT];
-            loadP(pv, j0);
+        for (int e = 0; e < EPT; ++e) s[e] = 0;
+        for (int j0 = 0; j0 < k; j0 += CH) {
+            if (k > CH) loadP(j0);
 #pragma unroll
-            for (int jj = 0; jj < kGroup; ++jj)
-                if (j0 + jj < k)
+            for (int i = 0; i < CH; ++i) {
+                const double u = L.u[j0 + i];  // 0 from k on
 #pragma unroll
-                    for (int i = 0; i < EPT; ++i) s[i] += (double)pv[jj][i] * sU[j0 + jj];
+                for (int e = 0; e < EPT; ++e) s[e] = fma((double)pv[i][e], u, s[e]);
+            }
         }
+        if (on)
 #pragma unroll
-        for (int i = 0; i < EPT; ++i)
-            if (nv[i]) p[i] -= s[i];
-        __syncthreads();
+            for (int e = 0; e < EPT; ++e) p[e] -= s[e];
     }
-    double v = 0;  // sum of squares in element order (the terms beyond ld are zero)
+    double v = 0;
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) v = i == 0 ? p[0] * p[0] : v + p[i] * p[i];
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) sW[wv][0] = v;
+    for (int e = 0; e < EPT; ++e) v = fma(p[e], p[e], v);
+    v = pca_row_sum(v);
+    if (l16 == 0) L.n[row] = v;
     __syncthreads();
-    double nrm2 = 0;
-    for (int w = 0; w < 16; ++w) nrm2 += sW[w][0];
-    const double inv = 1.0 / sqrt(nrm2);
+    // |p|^2 from the 64 rows' parts: each DPP row four apiece in order, then the row sum
+    double n2 = 0;
 #pragma unroll
-    for (int i = 0; i < EPT; ++i)
-        if (nv[i]) P[(long long)k * ld + tid + 1024 * i] = (float)(p[i] * inv);
+    for (int i = 0; i < 4; ++i) n2 += L.n[4 * l16 + i];
+    const double inv = 1.0 / sqrt(pca_row_sum(n2));
+    if (on) {
+        typedef float V __attribute__((ext_vector_type(EPT)));
+        V o;
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) o[e] = (float)(p[e] * inv);
+        *(V *)(P + (long long)k * ld + n0) = o;
+    }
 }
 
 extern "C" __global__ void __launch_bounds__(1024)
 PcaOrthonormalize(float *__restrict__ S, PCA_DIMS d) {
-    __shared__ double sW[16][PTK_PCA_MAX_K];
-    __shared__ double sU[PTK_PCA_MAX_K];
+    __shared__ PcaOrthoLds L;
     if (!pca_ok(d) || blockDim.x != 1024 || gridDim.x != 1) return;
-    if (d.ld <= 2048) pca_orthonormalize<2>(S, d, sW, sU);
-    else pca_orthonormalize<4>(S, d, sW, sU);
+    if (d.ld <= 2048) pca_orthonormalize<2>(S, d, L);
+    else pca_orthonormalize<4>(S, d, L);
 }
 
 // ---- PcaFinish: L_k = sqrt(sum of the G tn partials) (pca_cpu.cpp:385), one block of 256
