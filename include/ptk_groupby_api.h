@@ -4,8 +4,9 @@
  *
  * One call runs the same seven task kernels the groupby graph dispatches (GroupbyHistogram,
  * GroupbyBucketScan, GroupbyPartition, GroupbyKeyCount, GroupbyKeyScan, GroupbyReshuffle,
- * GroupbyTotals; layouts in ptk_groupby.h) on the caller's stream, in stream order, without synchronising.  Results are bitwise those of the
- * graph: per-key int64 counts and sums, the groups block {G, rows, errors, then G {key, count,
+ * GroupbyTotals; layouts in ptk_groupby.h) on the caller's stream, in stream order, without synchronising;
+ * up to 8192 rows one block orders them in LDS instead (one launch, or two over more than 4096 keys) and
+ * the workspace is not touched.  Results are bitwise those of the graph: per-key int64 counts and sums, the groups block {G, rows, errors, then G {key, count,
  * sum} in key order}, offsets, and the rows grouped by ascending key with the rows of a group in
  * input order.  Keys lie in [0, numKeys]; other keys are counted as errors and dropped.
  *

@@ -3,7 +3,8 @@
 //
 // The kernels are the graph's own (groupby.hip is compiled into this library unchanged), launched
 // on the caller's stream in the order the graph dispatches them, with the geometry the groupby
-// application gives its tasks.  Results are therefore bitwise the graph's.
+// application gives its tasks; up to GB_SMALL_ROWS rows one block does the whole of it in LDS
+// (groupby_small.h).  Results are bitwise the graph's.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -12,6 +13,7 @@
 #include <string>
 
 #include "groupby.hip"
+#include "groupby_small.h"
 #include "ptk_groupby_api.h"
 
 namespace {
@@ -36,9 +38,25 @@ bool ShapeOk(long long n, int numKeys) {
     return n >= 1 && n <= INT_MAX && numKeys >= 0 && (long long)numKeys + 1 <= PTK_GB_MAX_KEYS;
 }
 
-// The seven launches on `stream`; table and scratch lie in device memory the caller provides.
+// Few rows: one block, and one more launch when the offsets of many keys are to be written.
+template <int RPT>
+int LaunchSmall(const int *keys, const int *vals, int n, int numKeys, long long *offsets, long long *groups,
+                int *outKeys, int *outVals, hipStream_t stream) {
+    hipLaunchKernelGGL((GroupbySmall<RPT>), dim3(1), dim3(GB_SMALL_THREADS), 0, stream, keys, vals, n, numKeys, offsets,
+                       groups, outKeys, outVals);
+    if (numKeys >= GB_SMALL_KEYS)
+        hipLaunchKernelGGL(GroupbySmallOffsets, dim3((unsigned)(numKeys / 1024 + 1)), dim3(256), 0, stream,
+                           (const int *)outKeys, (const long long *)groups, numKeys, offsets);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? PTK_GB_OK : HipFail(e, "groupby launch");
+}
+
+// The launches on `stream`; table and scratch lie in device memory the caller provides.
 int Launch(const int *keys, const int *vals, int n, int numKeys, long long *table, void *scratch, long long *offsets,
            long long *groups, int *outKeys, int *outVals, hipStream_t stream) {
+    if (n <= 4 * GB_SMALL_THREADS) return LaunchSmall<4>(keys, vals, n, numKeys, offsets, groups, outKeys, outVals, stream);
+    if (n <= 4 * GB_SMALL_THREADS) return LaunchSmall<4>(keys, vals, n, numKeys, offsets, groups, outKeys, outVals, stream);
+    if (n <= GB_SMALL_ROWS) return LaunchSmall<GB_SMALL_RPT>(keys, vals, n, numKeys, offsets, groups, outKeys, outVals, stream);
     const unsigned chunks = (unsigned)ptk_gb_chunks(n), nb = (unsigned)ptk_gb_buckets(numKeys);
     const unsigned tiles = (unsigned)ptk_gb_tiles_max(n, numKeys);
     int cus = 256, dev = 0;
