@@ -96,6 +96,14 @@ PTK_GB_FN long long ptk_gb_buckets(int numKeys) {
 PTK_GB_FN long long ptk_gb_tiles_max(long long n, int numKeys) {
     return (n + PTK_GB_TILE - 1) / PTK_GB_TILE + ptk_gb_buckets(numKeys);
 }
+/* Blocks of a GroupbyPartition launch on `cus` compute units, two of which fit each: one per quarter
+ * chunk while all of those run at once (a grid of more blocks than chunks takes quarters), else up to
+ * one per chunk. */
+PTK_GB_FN unsigned int ptk_gb_part_grid(long long n, int cus) {
+    const long long chunks = ptk_gb_chunks(n), most = 2ll * (cus > 0 ? cus : 1);
+    const long long quarters = chunks * (PTK_GB_CHUNK / PTK_GB_SUB);
+    return (unsigned int)(quarters <= most ? quarters : chunks < most ? chunks : most);
+}
 PTK_GB_FN long long ptk_gb_align256(long long b) { return (b + 255) / 256 * 256; }
 
 /* Byte offsets of the scratch arrays, in layout order, and the total size (a multiple of 256). */

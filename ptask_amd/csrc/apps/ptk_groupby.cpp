@@ -212,7 +212,7 @@ int main(int argc, char **argv) {
         if (hip)
             if (Accelerator *acc = Runtime::GetAccelerator(ACCELERATOR_CLASS_HIP, 0))
                 if (acc->GetCoreCount()) cus = (int)acc->GetCoreCount();
-        const int partGrid = std::max(1, std::min(std::min(chunks, o.gbGrid), 2 * cus));
+        const int partGrid = std::max(1, std::min((int)ptk_gb_part_grid(n, cus), o.gbGrid));
         auto nk = [&](UINT i) {  // the sticky n and numKeys ports at formal indices i and i + 1
             return std::array<Port *, 2>{Runtime::CreatePort(STICKY_PORT, tInt, uid++, (char *)"n", i),
                                          Runtime::CreatePort(STICKY_PORT, tInt, uid++, (char *)"numKeys", i + 1)};

@@ -695,7 +695,7 @@ int IssuePlain(ptk_batch *B, const Inst &in) {
         t.ptr(d.scratch).add<int>(n).add<int>(nk).ptr(d.table).ptr(d.groups);
         if (int r = B->Launch(B->fPGb[0], chunks, 1, 1, PTK_GB_HIST_THREADS, h)) return r;
         if (int r = B->Launch(B->fPGb[1], nb, 1, 1, PTK_GB_SCAN_THREADS, b)) return r;
-        if (int r = B->Launch(B->fPGb[2], std::min(chunks, (unsigned)(2 * B->cus)), 1, 1, PTK_GB_PART_THREADS, p)) return r;
+        if (int r = B->Launch(B->fPGb[2], std::max(1u, ptk_gb_part_grid(d.n, B->cus)), 1, 1, PTK_GB_PART_THREADS, p)) return r;
         if (int r = B->Launch(B->fPGb[3], tiles, 1, 1, PTK_GB_COUNT_THREADS, k)) return r;
         if (int r = B->Launch(B->fPGb[4], 2 * nb, 1, 1, PTK_GB_KEYSCAN_THREADS, s)) return r;
         if (int r = B->Launch(B->fPGb[5], tiles, 1, 1, PTK_GB_TILE_THREADS, r6)) return r;

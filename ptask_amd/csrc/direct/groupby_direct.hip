@@ -62,7 +62,7 @@ int Launch(const int *keys, const int *vals, int n, int numKeys, long long *tabl
     int cus = 256, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         cus = 256;
-    const unsigned partGrid = std::min(chunks, (unsigned)(2 * std::max(cus, 1)));  // two blocks per CU
+    const unsigned partGrid = ptk_gb_part_grid(n, cus);
     hipLaunchKernelGGL(GroupbyHistogram, dim3(chunks), dim3(PTK_GB_HIST_THREADS), 0, stream, keys, n, numKeys, scratch);
     hipLaunchKernelGGL(GroupbyBucketScan, dim3(nb), dim3(PTK_GB_SCAN_THREADS), 0, stream, scratch, n, numKeys);
     hipLaunchKernelGGL(GroupbyPartition, dim3(partGrid), dim3(PTK_GB_PART_THREADS), 0, stream, keys, vals, n, numKeys,

@@ -52,6 +52,11 @@ GroupbyPartition(const int *__restrict__ keys, const int *__restrict__ vals, int
     const PTK_GB_SCRATCH S = ptk_gb_scratch(scratch, n, numKeys);
     if (blockIdx.x == 0) gb_partition_starts(S, L);
     const unsigned G = gridDim.x < S.chunks ? gridDim.x : (unsigned)S.chunks;
+    if (gridDim.x > S.chunks) {  // more blocks than chunks: a quarter chunk each
+        const unsigned nq = (unsigned)S.chunks * GB_PART_SUBS, Q = gridDim.x < nq ? gridDim.x : nq;
+        if (blockIdx.x < Q) gb_partition_quarters(keys, vals, n, numKeys, gb_xcd_block(blockIdx.x, Q), Q, S, L);
+        return;
+    }
     if (blockIdx.x >= G) return;
     gb_partition_chunks(keys, vals, n, numKeys, gb_xcd_block(blockIdx.x, G), S.chunks, G, S, L);
 }
