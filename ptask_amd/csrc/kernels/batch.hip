@@ -34,8 +34,8 @@
 #include "fdtd_halves.h"
 #include "gmm_body.h"
 #include "gmm_mfma.h"
-// the work-list loop costs the keyscan a few registers: 32 tiles per load batch keep it unspilled
-#define GB_KS_BATCH 32
+// the work-list loop costs the keyscan a few registers: 12 tiles per load batch keep it under 64, unspilled
+#define GB_KS_BATCH 12
 #include "groupby_body.h"
 #include "ptk_batch.h"
 #include "ptk_prng.h"
@@ -243,7 +243,7 @@ BatchGroupbyKeyCount(const int2 *__restrict__ units, const int *__restrict__ cou
 }
 
 // Units {inst, half bucket}.
-extern "C" __global__ void __launch_bounds__(PTK_GB_KEYSCAN_THREADS)
+extern "C" __global__ void __launch_bounds__(PTK_GB_KEYSCAN_THREADS, 8)
 BatchGroupbyKeyScan(const int2 *__restrict__ units, const int *__restrict__ count, const PTK_GROUPBY_INST *__restrict__ insts) {
     __shared__ GbKeyScanLds L;
     if (blockDim.x != PTK_GB_KEYSCAN_THREADS) return;

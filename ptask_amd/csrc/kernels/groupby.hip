@@ -70,7 +70,7 @@ extern "C" __global__ void __launch_bounds__(PTK_GB_COUNT_THREADS) GroupbyKeyCou
 }
 
 // Units of half a bucket (two per bucket); any grid.
-extern "C" __global__ void __launch_bounds__(PTK_GB_KEYSCAN_THREADS)
+extern "C" __global__ void __launch_bounds__(PTK_GB_KEYSCAN_THREADS, 8)
 GroupbyKeyScan(void *scratch, int n, int numKeys, long long *offsets) {
     __shared__ GbKeyScanLds L;
     if (!gb_keys_ok(numKeys) || n < 0 || blockDim.x != PTK_GB_KEYSCAN_THREADS) return;

@@ -507,8 +507,13 @@ __device__ inline void gb_keycount_tile(const PTK_GB_SCRATCH &S, unsigned t, GbK
 
 #define GB_KS_KEYS (PTK_GB_BUCKET / 2)                    // keys per keyscan block (half a bucket)
 #define GB_KS_PARTS (PTK_GB_KEYSCAN_THREADS / GB_KS_KEYS)    // threads per key in keyscan
+// Tiles whose counts a keyscan thread loads at once.  Sixteen leave the kernel under 64 registers, so
+// that two of its 1024-thread blocks fit a CU (the kernels ask for that): most buckets have a few tiles
+// and the launch lasts as long as its rounds of blocks.  Whole groupby, us, against forty tiles at once on
+// 110 registers: 1M rows over 262144 keys 77.5 (87.9), 500,000 over 65536 45.6 (48.4), 8M over 65536
+// 117.8 (118.5); and 8M over 16, whose one bucket has 1953 tiles, 222 (227).
 #ifndef GB_KS_BATCH
-#define GB_KS_BATCH 40  // tiles whose counts a keyscan thread loads at once
+#define GB_KS_BATCH 16
 #endif
 #define GB_TS_KEYS (PTK_GB_BUCKET / 4)                    // keys per totals block (a quarter bucket)
 #define GB_TS_PARTS (PTK_GB_TOTALS_THREADS / GB_TS_KEYS)     // threads per key in totals
