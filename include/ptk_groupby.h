@@ -97,12 +97,12 @@ PTK_GB_FN long long ptk_gb_tiles_max(long long n, int numKeys) {
     return (n + PTK_GB_TILE - 1) / PTK_GB_TILE + ptk_gb_buckets(numKeys);
 }
 /* Blocks of a GroupbyPartition launch on `cus` compute units, two of which fit each: one per quarter
- * chunk while all of those run at once (a grid of more blocks than chunks takes quarters), else up to
- * one per chunk. */
+ * chunk while they run in two rounds at most, else up to one per chunk, and one more for the starts and
+ * the tile table.  (A quarter takes 11 us, or 7 with a CU to itself: 3M rows 22 us against 28.) */
 PTK_GB_FN unsigned int ptk_gb_part_grid(long long n, int cus) {
     const long long chunks = ptk_gb_chunks(n), most = 2ll * (cus > 0 ? cus : 1);
     const long long quarters = chunks * (PTK_GB_CHUNK / PTK_GB_SUB);
-    return (unsigned int)(quarters <= most ? quarters : chunks < most ? chunks : most);
+    return (unsigned int)(quarters <= 2 * most ? quarters + 1 : chunks < most ? chunks + 1 : most);
 }
 PTK_GB_FN long long ptk_gb_align256(long long b) { return (b + 255) / 256 * 256; }
 

@@ -50,15 +50,23 @@ GroupbyPartition(const int *__restrict__ keys, const int *__restrict__ vals, int
     __shared__ GbPartLds L;
     if (!gb_keys_ok(numKeys) || n < 0 || blockDim.x != PTK_GB_PART_THREADS) return;
     const PTK_GB_SCRATCH S = ptk_gb_scratch(scratch, n, numKeys);
-    if (blockIdx.x == 0) gb_partition_starts(S, L);
-    const unsigned G = gridDim.x < S.chunks ? gridDim.x : (unsigned)S.chunks;
-    if (gridDim.x > S.chunks) {  // more blocks than chunks: a quarter chunk each
-        const unsigned nq = (unsigned)S.chunks * GB_PART_SUBS, Q = gridDim.x < nq ? gridDim.x : nq;
-        if (blockIdx.x < Q) gb_partition_quarters(keys, vals, n, numKeys, gb_xcd_block(blockIdx.x, Q), Q, S, L);
-        return;
+    // Units: quarter chunks when the grid has a block for each, else chunks.  The starts and the tile
+    // table, which nothing in this launch reads, are one block's: one of its own where the grid has one
+    // to spare or the others need no more rounds without it, else block 0.
+    const bool quarters = gridDim.x >= S.chunks * GB_PART_SUBS;
+    const unsigned units = (unsigned)S.chunks * (quarters ? GB_PART_SUBS : 1);
+    unsigned G = gridDim.x < units ? gridDim.x : units, b = blockIdx.x;
+    if (gridDim.x > units) {
+        if (b == units) gb_partition_starts(S, L);
+    } else if (G > 1 && (units + G - 2) / (G - 1) == (units + G - 1) / G) {
+        if (b == 0) gb_partition_starts(S, L);
+        --G, b = b == 0 ? ~0u : b - 1;
+    } else if (b == 0) {
+        gb_partition_starts(S, L);
     }
-    if (blockIdx.x >= G) return;
-    gb_partition_chunks(keys, vals, n, numKeys, gb_xcd_block(blockIdx.x, G), S.chunks, G, S, L);
+    if (b >= G) return;
+    if (quarters) gb_partition_quarters(keys, vals, n, numKeys, gb_xcd_block(b, G), G, S, L);
+    else gb_partition_chunks(keys, vals, n, numKeys, gb_xcd_block(b, G), S.chunks, G, S, L);
 }
 
 extern "C" __global__ void __launch_bounds__(PTK_GB_COUNT_THREADS) GroupbyKeyCount(void *scratch, int n, int numKeys) {

@@ -127,11 +127,39 @@ __device__ inline unsigned long long gb_match(unsigned d, bool use) {
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// The same for an 8-bit digit through LDS: each lane ORs its bit into the word of its digit and reads the
+// word back.  `mask` is the wave's own 256 words, zero on entry and on return; nothing else orders the
+// lanes (the LDS instructions of a wave complete in order, and OR does not depend on it).  The lanes that
+// share the first lane's digit are found with one ballot and stay out of it: where one key dominates, most
+// lanes would meet in one word, which takes them one at a time.
+__device__ __forceinline__ unsigned long long gb_match_lds(unsigned d, bool use, unsigned long long *mask) {
+    const unsigned long long on = __ballot(use);
+    if (on == 0) return 0;
+    const unsigned d0 = (unsigned)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(on));
+    const unsigned long long same = __ballot(use && d == d0);
+    unsigned long long peers = same;
+    if (use && d != d0) {
+        unsigned long long *const w = mask + d;
+        __hip_atomic_fetch_or(w, 1ull << (threadIdx.x & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        peers = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __hip_atomic_store(w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    return peers;
+}
+
 #define GB_HIST_WAVES (PTK_GB_HIST_THREADS / 64)
 #define GB_HIST_ROWS (PTK_GB_CHUNK / PTK_GB_HIST_THREADS)  // rows per thread (16)
 
+// Counters of the histogram: lanes l, l + 8, .. of a wave share one copy of the bucket counts, so that rows
+// of one bucket meet an eighth as often in one address (LDS atomics on one address are taken one at a
+// time).  Copies start on different banks (an odd stride); more than GB_HIST_COPIED buckets have one copy.
+#define GB_HIST_COPIED 256
+#define GB_HIST_COPIES 8
 struct GbHistLds {
-    unsigned cnt[PTK_GB_MAX_BUCKETS];  // per bucket: rows of the chunk
+    union {
+        unsigned one[PTK_GB_MAX_BUCKETS];
+        unsigned copy[GB_HIST_COPIES][GB_HIST_COPIED + 1];
+    } cnt;
     unsigned long long red[16];
 };
 
@@ -168,8 +196,11 @@ __device__ inline void gb_histogram_chunk(const int *__restrict__ keys, long lon
                                           const PTK_GB_SCRATCH &S, GbHistLds &L) {
     const int NB = (int)S.buckets, tid = threadIdx.x;
     const long long r0 = c * PTK_GB_CHUNK, nr = n - r0 < PTK_GB_CHUNK ? n - r0 : PTK_GB_CHUNK;
+    const bool copied = NB <= GB_HIST_COPIED;
+    unsigned *const mine = copied ? L.cnt.copy[tid % GB_HIST_COPIES] : L.cnt.one;
+    const int words = copied ? GB_HIST_COPIES * (GB_HIST_COPIED + 1) : NB;
     __syncthreads();
-    for (int b = tid; b < NB; b += PTK_GB_HIST_THREADS) L.cnt[b] = 0;
+    for (int b = tid; b < words; b += PTK_GB_HIST_THREADS) L.cnt.one[b] = 0;
     int4 kv[GB_HIST_ROWS / 4];
     const int4 *k4 = (const int4 *)(keys + r0);  // r0 is a multiple of 4: 16-byte aligned
     unsigned inRange = GB_HIST_ROWS;
@@ -192,7 +223,7 @@ __device__ inline void gb_histogram_chunk(const int *__restrict__ keys, long lon
     unsigned good = 0;
     auto add = [&](int k) {
         if (k >= 0 && k <= numKeys) {
-            atomicAdd(&L.cnt[(unsigned)k / PTK_GB_BUCKET], 1u);
+            atomicAdd(&mine[(unsigned)k / PTK_GB_BUCKET], 1u);
             ++good;
         }
     };
@@ -206,7 +237,16 @@ __device__ inline void gb_histogram_chunk(const int *__restrict__ keys, long lon
     const unsigned err = inRange - good;
     __syncthreads();
     unsigned *h = S.hist + c * NB;
-    for (int b = tid; b < NB; b += PTK_GB_HIST_THREADS) h[b] = L.cnt[b];
+    for (int b = tid; b < NB; b += PTK_GB_HIST_THREADS) {
+        unsigned t = 0;
+        if (copied) {
+#pragma unroll
+            for (int i = 0; i < GB_HIST_COPIES; ++i) t += L.cnt.copy[i][b];
+        } else {
+            t = L.cnt.one[b];
+        }
+        h[b] = t;
+    }
     const unsigned long long e = block_sum(err, L.red);
     if (tid == 0) S.berr[c] = (unsigned)e;
     __syncthreads();
@@ -244,6 +284,10 @@ __device__ inline void gb_bucketscan(const PTK_GB_SCRATCH &S, int b, unsigned *r
 struct GbPartLds {
     union {
         unsigned short wcnt[GB_PART_WAVES][PTK_GB_MAX_BUCKETS];  // per wave and bucket: rows, then the wave's base
+        struct {                                                  // up to 256 buckets
+            unsigned short wcnt[GB_PART_WAVES][256];
+            unsigned long long match[GB_PART_WAVES][256];         // gb_match_lds
+        } n;
         int2 stage[PTK_GB_SUB];  // once the rows are ranked: {key, value} in partitioned order
     } u;
     unsigned dest[PTK_GB_MAX_BUCKETS];  // per bucket: the partitioned row of the chunk's next row of the bucket
@@ -282,12 +326,19 @@ __device__ inline void gb_partition_starts(const PTK_GB_SCRATCH &S, GbPartLds &L
     for (long long c = tid; c < S.chunks; c += blockDim.x) err += S.berr[c];
     err = block_sum(err, L.red64);
     if (tid == 0) S.head[0] = err;
-    for (int b = tid; b < NB; b += blockDim.x) {  // the tile table: bucket, first and end row
-        const unsigned r0 = L.base[b], end = r0 + S.btot[b], t0 = ts[b], t1 = ts[b + 1];
-        for (unsigned t = t0; t < t1; ++t) {
-            const unsigned a = r0 + (t - t0) * PTK_GB_TILE;
-            *(uint4 *)(S.tinfo + 4ull * t) = make_uint4((unsigned)b, a, a + PTK_GB_TILE < end ? a + PTK_GB_TILE : end, 0u);
+    // the tile table: bucket, first and end row.  A thread per tile, which finds its bucket among the
+    // tile starts: a bucket may have one tile or all of them (8M rows of one bucket: 1953 tiles, 45 us
+    // when a thread wrote a bucket's).
+    const unsigned nt = ts[NB];
+    for (unsigned t = tid; t < nt; t += blockDim.x) {
+        int lo = 0, hi = NB;  // ts[lo] <= t < ts[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (ts[mid] <= t) lo = mid;
+            else hi = mid;
         }
+        const unsigned a = L.base[lo] + (t - ts[lo]) * PTK_GB_TILE, end = lo + 1 < NB ? L.base[lo + 1] : rows;
+        *(uint4 *)(S.tinfo + 4ull * t) = make_uint4((unsigned)lo, a, a + PTK_GB_TILE < end ? a + PTK_GB_TILE : end, 0u);
     }
     __syncthreads();
 }
@@ -311,6 +362,7 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
     int q = 0;
     if (QUARTERS) q = (int)(c % GB_PART_SUBS), c /= GB_PART_SUBS, cend = S.chunks;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto wcnt = [&](int v, unsigned b) -> unsigned short & { return BITS == 8 ? L.u.n.wcnt[v][b] : L.u.wcnt[v][b]; };
     __syncthreads();
     for (int b = tid; b < NB; b += PTK_GB_PART_THREADS) L.bst[b] = S.btot[b];
     gb_lds_exscan(L.bst, NB, L.red);  // bucket starts
@@ -354,8 +406,12 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
             const long long row0 = c * PTK_GB_CHUNK + (long long)q * PTK_GB_SUB;
             const long long wr0 = row0 + (long long)w * (PTK_GB_SUB / GB_PART_WAVES);
             const int nin = wr0 >= n ? 0 : (n - wr0 < 64 * GB_PART_ROWS ? (int)(n - wr0) : 64 * GB_PART_ROWS);
-            for (int v = 0; v < GB_PART_WAVES; ++v)
-                for (int b = tid; b < NB; b += PTK_GB_PART_THREADS) L.u.wcnt[v][b] = 0;
+            if (BITS == 8) {
+                for (int i = tid; i < (int)sizeof(L.u.n) / 16; i += PTK_GB_PART_THREADS) ((uint4 *)&L.u.n)[i] = make_uint4(0, 0, 0, 0);
+            } else {
+                for (int v = 0; v < GB_PART_WAVES; ++v)
+                    for (int b = tid; b < NB; b += PTK_GB_PART_THREADS) wcnt(v, b) = 0;
+            }
             __syncthreads();
             // ranks in row order: wave w, step s covers 64 consecutive rows; rk: the rank among the
             // wave's rows of the bucket, then the row's position in the quarter's partitioned order
@@ -365,10 +421,10 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
             for (int s = 0; s < GB_PART_ROWS; ++s) {
                 const bool use = 64 * s + lane < nin && kr[s] >= 0 && kr[s] <= numKeys;
                 const unsigned d = use ? (unsigned)kr[s] / PTK_GB_BUCKET : 0u;
-                const unsigned long long peers = gb_match<BITS>(d, use);
+                const unsigned long long peers = BITS == 8 ? gb_match_lds(d, use, L.u.n.match[w]) : gb_match<BITS>(d, use);
                 unsigned old = 0;
-                if (use) old = L.u.wcnt[w][d];
-                if (use && (peers & below) == 0) L.u.wcnt[w][d] = (unsigned short)(old + __popcll(peers));
+                if (use) old = wcnt(w, d);
+                if (use && (peers & below) == 0) wcnt(w, d) = (unsigned short)(old + __popcll(peers));
                 rk[s] = use ? old + (unsigned)__popcll(peers & below) : 0xFFFFFFFFu;
                 __builtin_amdgcn_sched_barrier(0);  // one step at a time: keeps the ballots' masks few
             }
@@ -377,8 +433,8 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
                 unsigned t = 0;
 #pragma unroll
                 for (int v = 0; v < GB_PART_WAVES; ++v) {
-                    const unsigned x = L.u.wcnt[v][b];
-                    L.u.wcnt[v][b] = (unsigned short)t;
+                    const unsigned x = wcnt(v, b);
+                    wcnt(v, b) = (unsigned short)t;
                     t += x;
                 }
                 L.base[b] = t;
@@ -389,7 +445,7 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
             for (int s = 0; s < GB_PART_ROWS; ++s) {
                 if (rk[s] == 0xFFFFFFFFu) continue;
                 const unsigned d = (unsigned)kr[s] / PTK_GB_BUCKET;
-                rk[s] += L.base[d] + L.u.wcnt[w][d];
+                rk[s] += L.base[d] + wcnt(w, d);
             }
             __syncthreads();
             // per bucket: the partitioned row of local position 0, and the next quarter's start
@@ -602,6 +658,7 @@ __device__ inline void gb_keyscan_half(const PTK_GB_SCRATCH &S, int numKeys, int
 }
 
 #define GB_TILE_WAVES (PTK_GB_TILE_THREADS / 64)
+static_assert(PTK_GB_TILE_THREADS >= PTK_GB_BUCKET, "a reshuffle block has a thread per key");
 #define GB_TILE_ROWS (PTK_GB_TILE / PTK_GB_TILE_THREADS)  // rows per thread (8)
 
 struct GbShuffleLds {
@@ -638,6 +695,11 @@ __device__ inline void gb_reshuffle_tiles(const PTK_GB_SCRATCH &S, int numKeys, 
         const unsigned rows = T.r1 - T.r0;
         const long long wr0 = (long long)T.r0 + (long long)w * (PTK_GB_TILE / GB_TILE_WAVES);
         const int nin = wr0 >= T.r1 ? 0 : (T.r1 - wr0 < 64 * GB_TILE_ROWS ? (int)(T.r1 - wr0) : 64 * GB_TILE_ROWS);
+        // key tid's first output row of the tile, loaded while the rows are ranked
+        const long long key0 = (long long)T.bucket * PTK_GB_BUCKET;
+        long long out0 = 0;
+        if (tid < PTK_GB_BUCKET && key0 + tid <= numKeys)  // keys past numKeys have no rows
+            out0 = offsets[key0 + tid] + (long long)S.c2[(unsigned long long)t * PTK_GB_BUCKET + tid];
         __syncthreads();
         for (int q = 0; q < GB_TILE_WAVES; ++q)
             for (int k = tid; k < PTK_GB_BUCKET; k += PTK_GB_TILE_THREADS) L.wcnt[q][k] = 0;
@@ -668,12 +730,7 @@ __device__ inline void gb_reshuffle_tiles(const PTK_GB_SCRATCH &S, int numKeys, 
             L.start[k] = tt;
         }
         gb_lds_exscan(L.start, PTK_GB_BUCKET, L.red);
-        const long long key0 = (long long)T.bucket * PTK_GB_BUCKET;
-        const unsigned *c2 = S.c2 + (unsigned long long)t * PTK_GB_BUCKET;
-        for (int k = tid; k < PTK_GB_BUCKET; k += PTK_GB_TILE_THREADS) {
-            const long long o = key0 + k <= numKeys ? offsets[key0 + k] : 0;  // keys past numKeys have no rows
-            L.base[k] = (int)(o + (long long)c2[k] - (long long)L.start[k]);
-        }
+        if (tid < PTK_GB_BUCKET) L.base[tid] = (int)(out0 - (long long)L.start[tid]);
 #pragma unroll
         for (int s = 0; s < GB_TILE_ROWS; ++s) {
             if (rk[s] == 0xFFFFFFFFu) continue;
