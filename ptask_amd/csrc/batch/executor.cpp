@@ -336,7 +336,11 @@ int Admit(ptk_batch *B, Inst &in) {
         const unsigned long long K = (unsigned long long)in.b + 1;
         d.n = in.a;
         d.numKeys = in.b;
-        d.chunkRows = B->gbRows;
+        // At most gbRows rows per unit, and sixteen units where the rows allow it: a unit's chunks are
+        // taken one after the other, and a few instances would leave most CUs without one.  12
+        // instances of 2,000 to 1,000,000 rows over 4096 keys: 0.54 -> 0.25 ms in all (units of 262144
+        // rows before); 100 of them, which fill the chip either way: 0.91 -> 0.84.
+        d.chunkRows = (int)std::min<long long>(B->gbRows, std::max(1LL, (ptk_gb_chunks(in.a) + 15) / 16) * PTK_GB_CHUNK);
         d.keys = (const int *)carve(4ull * in.a);
         d.vals = (const int *)carve(4ull * in.a);
         d.outKeys = (int *)carve(4ull * in.a);
