@@ -301,18 +301,22 @@ __device__ inline void gmm_finalize_block(double *__restrict__ model, const doub
             const long long col = c == 0   ? (long long)k
                                   : c <= D ? K + (long long)k * D + (c - 1)
                                            : K + (long long)K * D + (long long)k * D + (c - 1 - D);
-            // rows g, g + G, ... in order; sixteen rows' loads issued together (a row past the
-            // last reads row g and is not added)
+            // rows g, g + G, ... in order; kRows rows' loads issued together (a row past the
+            // last reads row g and is not added).  A serial chain of round trips to memory: sixteen
+            // rows at a time took 15.3 us over 768 rows (D = 32, K = 64) and 6.9 over 391 (D = 16,
+            // K = 24), 32 take 12.8 and 6.4, 64 take 13.2 and 6.5.
+            constexpr int kRows = 32;
             const double *src = partials + col;
-            for (int b0 = g; b0 < P; b0 += 16 * G) {
-                double v[16];
+            for (int b0 = g; b0 < P; b0 += kRows * G) {
+                double v[kRows];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) {
+                for (int u = 0; u < kRows; ++u) {
                     const int b = b0 + u * G;
                     v[u] = src[(long long)(b < P ? b : g) * S];
                 }
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
+                for (int u = 0; u < kRows; ++u)
                     if (b0 + u * G < P) acc += v[u];
             }
         }
