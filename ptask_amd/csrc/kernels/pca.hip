@@ -28,6 +28,8 @@
 // Tolerance-checked binary32 work: let the compiler fuse multiply-adds (the build default is off).
 #pragma clang fp contract(fast)
 
+#define PCA_LOAD_COLS 128  // columns of a tile of PcaLoad
+
 enum { PCA_START = 0, PCA_GRAM = 1, PCA_DEFLATE = 3 };
 
 __device__ inline bool pca_ok(const PCA_DIMS &d) {
@@ -46,69 +48,69 @@ __device__ inline float f4get(const float4 &v, int e) { return e == 0 ? v.x : e 
 __device__ inline float f4dot(const float4 &a, const float4 &b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
 
 // ---- PcaLoad: X (column-major M x N) -> R (row-major Mp x ld), rows optionally centred; T and S
-// cleared.  Grid Mp/64 blocks of 256; block b owns rows 64b .. 64b+63.
+// cleared.  Grid Mp/64 blocks of 256; block b owns rows 64b .. 64b+63.  With few rows only some CUs
+// have a block and the time is its chain of round trips and address arithmetic: 32 loads in flight
+// per thread from scalar column addresses take 24.3 us at 3000 x 700 (8 and 16 from per-lane 64-bit
+// products took 39.0, and 64 in flight give no more); at 65536 x 2048 it is two reads and a write of
+// the matrix at 4.5 TB/s, 359 us, as before.
 extern "C" __global__ void __launch_bounds__(256)
 PcaLoad(const float *__restrict__ X, PCA_DIMS d, float *__restrict__ R, float *__restrict__ T,
         float *__restrict__ S) {
     __shared__ double sSum[4][64];
     __shared__ double sMean[64];
-    __shared__ float tile[64][65];
+    __shared__ float tile[PCA_LOAD_COLS][65];
     if (!pca_ok(d) || blockDim.x != 256 || (int)gridDim.x != d.Mp / 64) return;
     const int tid = threadIdx.x, M = d.M, N = d.N, ld = d.ld;
     const long long r0 = (long long)blockIdx.x * 64;
+    // Column c0 + 4 j is one wave's, row r one lane's: a column's address is a scalar, the lane's
+    // offset from it the same 32 bits in every load (the rows past the last read the last).
+    const int r = tid & 63, c0 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned ro = (unsigned)(r0 + r < M ? r : M - 1 - r0);
+    const bool mv = r0 + r < M;
+    constexpr int kLoads = PCA_LOAD_COLS / 4;
+    float v[kLoads];
+    auto load = [&](int n0) {  // columns n0 + c0 + 4 j; past the last, the last
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int n = n0 + c0 + 4 * j;
+            v[j] = (X + ((long long)(n < N ? n : N - 1) * M + r0))[ro];
+        }
+    };
+    load(0);
     {
-        // row sums: eight columns' loads issued together (row and column indexes clamped in
-        // range), added in column order
-        const int r = tid & 63, grp = tid >> 6;
-        const long long m = r0 + r < M ? r0 + r : M - 1;
+        // row sums, added in column order
         double s = 0;
-        if (d.center && r0 + r < M)
-            for (int n0 = grp; n0 < N; n0 += 32) {
-                float v[8];
+        if (d.center)
+            for (int n0 = 0; n0 < N; n0 += PCA_LOAD_COLS) {
+                if (n0 > 0) load(n0);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int n = n0 + 4 * u < N ? n0 + 4 * u : N - 1;
-                    v[u] = X[(long long)n * M + m];
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (n0 + 4 * u < N) s += (double)v[u];
+                for (int j = 0; j < kLoads; ++j)
+                    if (n0 + c0 + 4 * j < N) s += (double)v[j];
             }
-        sSum[grp][r] = s;
+        sSum[c0][r] = s;
     }
+    if (d.center && N > PCA_LOAD_COLS) load(0);
     __syncthreads();
     if (tid < 64) sMean[tid] = d.center ? (sSum[0][tid] + sSum[1][tid] + sSum[2][tid] + sSum[3][tid]) / N : 0.0;
     __syncthreads();
-    // 64 x 64 tiles through LDS; the next tile's sixteen loads per thread are issued before the
-    // current tile is transposed and stored
-    const int r = tid & 63, c0 = tid >> 6;
-    const long long m = r0 + r < M ? r0 + r : M - 1;
-    const bool mv = r0 + r < M;
-    float cur[16], nxt[16];
-    auto load = [&](float (&v)[16], int n0) {
+    // 64 x PCA_LOAD_COLS tiles through LDS; the next tile's loads are issued before the current tile
+    // is stored
+    const double mean = sMean[r];
+    const int w0 = __builtin_amdgcn_readfirstlane(tid / PCA_LOAD_COLS), wc = tid % PCA_LOAD_COLS;
+    for (int n0 = 0; n0 < ld; n0 += PCA_LOAD_COLS) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int n = n0 + c0 + 4 * j;
-            v[j] = X[(long long)(n < N ? n : N - 1) * M + m];
-        }
-    };
-    load(cur, 0);
-    for (int n0 = 0; n0 < ld; n0 += 64) {
-        if (n0 + 64 < ld) load(nxt, n0 + 64);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        for (int j = 0; j < kLoads; ++j) {
             const int c = c0 + 4 * j;
-            tile[c][r] = (n0 + c < N && mv) ? (float)((double)cur[j] - sMean[r]) : 0.f;
+            tile[c][r] = (n0 + c < N && mv) ? (float)((double)v[j] - mean) : 0.f;
         }
         __syncthreads();
-        for (int i = tid; i < 64 * 64; i += 256) {
-            const int rr = i >> 6, c = i & 63;
-            if (n0 + c < ld) R[(r0 + rr) * ld + n0 + c] = tile[c][rr];
-        }
+        if (n0 + PCA_LOAD_COLS < ld) load(n0 + PCA_LOAD_COLS);
+        __builtin_amdgcn_sched_barrier(0);
+        if (n0 + wc < ld)
+#pragma unroll 8
+            for (int rr = w0; rr < 64; rr += 256 / PCA_LOAD_COLS) (R + ((r0 + rr) * ld + n0))[(unsigned)wc] = tile[wc][rr];
         __syncthreads();
-        if (n0 + 64 < ld)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) cur[j] = nxt[j];
     }
     const long long nT = (long long)d.K * d.Mp, nS = ptk_pca_state_bytes(&d) / 4;
     const long long step = (long long)gridDim.x * 256;
