@@ -153,8 +153,8 @@ struct ptk_batch {
     ptk_hip_function fH = nullptr, fE = nullptr, fStep = nullptr, fStep3 = nullptr, fAdv = nullptr, fGbHist = nullptr,
                      fGbBScan = nullptr, fGbPart = nullptr, fGbKCount = nullptr, fGbKScan = nullptr, fGbRes = nullptr,
                      fGbTot = nullptr, fGmmAcc = nullptr, fGmmFin = nullptr, fInitFdtd = nullptr,
-                     fInitGb = nullptr, fInitGmm = nullptr, fInitGmmModel = nullptr, fSumWords = nullptr,
-                     fSumPairs = nullptr, fSumGroups = nullptr, fSumJobs = nullptr, fFill = nullptr;
+                     fInitGb = nullptr, fInitGmm = nullptr, fInitGmmModel = nullptr, fSumJobs = nullptr,
+                     fFill = nullptr;
     ptk_hip_function fSix[6] = {}, fPGb[7] = {},  // the groupby graph's seven kernels, in order
                      fPGmmAcc = nullptr, fPGmmFin = nullptr;
     void *arenaBase = nullptr;
@@ -823,9 +823,7 @@ int ptk_batch_create(const char *kernel_dir, unsigned long long arena_bytes, int
         {&B->fGbKScan, "BatchGroupbyKeyScan"}, {&B->fGbRes, "BatchGroupbyReshuffle"}, {&B->fGbTot, "BatchGroupbyTotals"},
         {&B->fGmmAcc, "BatchGmmAccumulateMfma"}, {&B->fGmmFin, "BatchGmmFinalize"},
         {&B->fInitFdtd, "BatchInitFdtd"}, {&B->fInitGb, "BatchInitGroupby"}, {&B->fInitGmm, "BatchInitGmm"},
-        {&B->fInitGmmModel, "BatchInitGmmModel"}, {&B->fSumWords, "BatchChecksumWords"},
-        {&B->fSumPairs, "BatchChecksumPairs"}, {&B->fSumGroups, "BatchChecksumGroups"},
-        {&B->fSumJobs, "BatchChecksumJobs"}};
+        {&B->fInitGmmModel, "BatchInitGmmModel"}, {&B->fSumJobs, "BatchChecksumJobs"}};
     for (auto &f : bf)
         if ((r = Load(B->mBatch, f.second, f.first))) return fail(r);
     static const char *six[6] = {"HxComputation", "HyComputation", "HzComputation",

@@ -431,58 +431,39 @@ BatchInitGmmModel(double *__restrict__ model, GMM_DIMS d, const float *__restric
 
 // ---- checksums --------------------------------------------------------------------------------
 
-__device__ inline void csum_add(unsigned long long *out, unsigned long long h) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) h += __shfl_xor(h, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out, h);
-}
-
-// sum over i of mix(bits(a[i]), i): changes with any bit and any position of the array.
-extern "C" __global__ void __launch_bounds__(256)
-BatchChecksumWords(const unsigned *__restrict__ a, long long n, unsigned long long *out) {
-    unsigned long long h = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        h += ptk_splitmix64(((unsigned long long)a[i] << 32) ^ (unsigned long long)i * 0x9E3779B97F4A7C15ull);
-    csum_add(out, h);
-}
-
 // All checksums of a set of retiring instances in one launch: grid (stripes, jobs); blocks of
-// job y stride over its elements.  Mode 2 (a groupby groups block) sums the header and the
-// G = groups[0] triples it holds; the rest of the block is never written and is not part of the
-// result.
+// job y stride over its elements, 2048 per block and turn.  Mode 2 (a groupby groups block) sums the
+// header and the G = groups[0] triples it holds; the rest of the block is never written and is not
+// part of the result.
+// The additions to a job's one word follow each other in memory, so a job of few elements takes few
+// blocks, and a block adds once; a thread's eight loads are in flight together.  24 FDTD instances of
+// 16^3 to 40^3: 11 us (52 with an addition per wave of 64 blocks and one load at a time).
 extern "C" __global__ void __launch_bounds__(256)
 BatchChecksumJobs(const PTK_CSUM_JOB *__restrict__ jobs) {
+    constexpr int kPer = 8, kTurn = 256 * kPer;
+    __shared__ unsigned long long sum[4];
     const PTK_CSUM_JOB J = jobs[blockIdx.y];
     const long long n = J.mode == 2 ? 2 * (3 + 3 * ((const long long *)J.a)[0]) : J.n;
-    const unsigned *a = (const unsigned *)J.a;
-    const int *k = (const int *)J.a, *v = (const int *)J.b;
+    if ((long long)blockIdx.x * kTurn >= n) return;
+    const unsigned *__restrict__ a = (const unsigned *)J.a, *__restrict__ v = (const unsigned *)J.b;
     unsigned long long h = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    for (long long i0 = (long long)blockIdx.x * kTurn + threadIdx.x; i0 < n; i0 += (long long)gridDim.x * kTurn) {
+        unsigned x[kPer], y[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) x[u] = a[min(i0 + 256 * u, n - 1)];
         if (J.mode == 1)
-            h += ptk_splitmix64(((unsigned long long)(unsigned)k[i] << 32) | (unsigned)v[i]);
-        else
-            h += ptk_splitmix64(((unsigned long long)a[i] << 32) ^ (unsigned long long)i * 0x9E3779B97F4A7C15ull);
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) y[u] = v[min(i0 + 256 * u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const long long i = i0 + 256 * u;
+            const unsigned long long low = J.mode == 1 ? (unsigned long long)y[u] : (unsigned long long)i * 0x9E3779B97F4A7C15ull;
+            const unsigned long long m = ptk_splitmix64(((unsigned long long)x[u] << 32) ^ low);
+            h += i < n ? m : 0ull;
+        }
     }
-    csum_add(J.out, h);
-}
-
-// The groups block of a groupby result: its header and the G = groups[0] triples it holds (the
-// rest of the block is never written and is not part of the result).
-extern "C" __global__ void __launch_bounds__(256)
-BatchChecksumGroups(const long long *__restrict__ groups, unsigned long long *out) {
-    const long long n = 2 * (3 + 3 * groups[0]);
-    const unsigned *a = (const unsigned *)groups;
-    unsigned long long h = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        h += ptk_splitmix64(((unsigned long long)a[i] << 32) ^ (unsigned long long)i * 0x9E3779B97F4A7C15ull);
-    csum_add(out, h);
-}
-
-// sum over rows of mix(key, value): the multiset of (key, value) pairs, independent of order.
-extern "C" __global__ void __launch_bounds__(256)
-BatchChecksumPairs(const int *__restrict__ k, const int *__restrict__ v, long long n, unsigned long long *out) {
-    unsigned long long h = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        h += ptk_splitmix64(((unsigned long long)(unsigned)k[i] << 32) | (unsigned)v[i]);
-    csum_add(out, h);
+    for (int off = 32; off >= 1; off >>= 1) h += __shfl_xor(h, off, 64);
+    if ((threadIdx.x & 63) == 0) sum[threadIdx.x >> 6] = h;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(J.out, sum[0] + sum[1] + sum[2] + sum[3]);
 }
