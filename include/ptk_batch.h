@@ -64,6 +64,13 @@ typedef struct _ptk_gmm_inst {
     GMM_DIMS d;
 } PTK_GMM_INST;
 
+/* FDTD instances admitted together, initialised by one launch (BatchInitFdtd). */
+#define PTK_INIT_FDTD_MAX 32
+typedef struct _ptk_init_fdtd {
+    int inst[PTK_INIT_FDTD_MAX];
+    unsigned long long seed[PTK_INIT_FDTD_MAX];
+} PTK_INIT_FDTD;
+
 /* One checksum of a retiring instance's result array (BatchChecksumJobs): mode 0 the words of
  * a[0..n), mode 1 the (key, value) pairs (a[i], b[i]), mode 2 a groupby groups block (its
  * length read from its header); the sum is added to *out. */

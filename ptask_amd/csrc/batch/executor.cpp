@@ -307,7 +307,28 @@ int EnsureCdf(ptk_batch *B, int numKeys, double s, long long *A) {
     return PTK_BATCH_OK;
 }
 
-// Places an instance's datablocks in the arena and generates its inputs on the device.
+// Generates the inputs of FDTD instances placed by Admit, up to PTK_INIT_FDTD_MAX per launch.
+int InitFdtd(ptk_batch *B, const std::vector<int> &ids) {
+    for (size_t i0 = 0; i0 < ids.size(); i0 += PTK_INIT_FDTD_MAX) {
+        PTK_INIT_FDTD J{};
+        const size_t n = std::min<size_t>(PTK_INIT_FDTD_MAX, ids.size() - i0);
+        long long elems = 1;
+        for (size_t i = 0; i < n; ++i) {
+            const Inst &in = B->insts[(size_t)ids[i0 + i]];
+            J.inst[i] = in.slot;
+            J.seed[i] = in.seed;
+            elems = std::max(elems, (in.a + 1) * (long long)(in.b + 1) * (in.c + 1));
+        }
+        Args a;
+        a.ptr(B->dFdtd).add(J);
+        const unsigned stripes = (unsigned)std::min(512ll, (elems + 255) / 256);
+        if (int r = B->Launch(B->fInitFdtd, stripes, (unsigned)n, 1, 256, a)) return r;
+    }
+    return PTK_BATCH_OK;
+}
+
+// Places an instance's datablocks in the arena and generates its inputs on the device (those of an
+// FDTD instance: InitFdtd, for all that are admitted together).
 int Admit(ptk_batch *B, Inst &in) {
     char *base = (char *)B->arenaBase + in.off;
     unsigned long long o = 0;
@@ -326,9 +347,6 @@ int Admit(ptk_batch *B, Inst &in) {
         d.steps = in.steps;
         d.done = 0;
         HIPCHK(ptk_hip_memcpy_htod_async(B->dFdtd + in.slot, &d, sizeof(d), B->stream));
-        Args a;
-        a.ptr(B->dFdtd).add<int>(in.slot).add<unsigned long long>(in.seed);
-        if (int r = B->Launch(B->fInitFdtd, 512, 1, 1, 256, a)) return r;
     } else if (in.kind == PTK_INST_GROUPBY) {
         in.slot = PopSlot(B->freeGb);
         if (in.slot < 0) return Fail(PTK_BATCH_ENOMEM, "too many resident groupby instances");
@@ -943,17 +961,21 @@ int ptk_batch_run(ptk_batch *B, int max_admit, int max_iters, int *niters, int *
     // admission: in submission order while the footprint fits
     int admitted = 0;
     size_t qi = 0;
+    std::vector<int> fdtd;
     while (qi < B->queue.size() && (max_admit < 0 || admitted < max_admit)) {
         Inst &in = B->insts[(size_t)B->queue[qi]];
         if (!B->arena.Alloc(in.bytes, &in.off)) break;
         if (int r = Admit(B, in)) {
             B->arena.Free(in.off, in.bytes);
+            InitFdtd(B, fdtd);
             return r;
         }
+        if (in.kind == PTK_INST_FDTD) fdtd.push_back(in.id);
         B->active.push_back(in.id);
         ++admitted;
         ++qi;
     }
+    if (int r = InitFdtd(B, fdtd)) return r;
     B->queue.erase(B->queue.begin(), B->queue.begin() + (long)qi);
     if (admitted) B->dirty = true;
     if (!B->active.empty() && B->mode == PTK_BATCH_BATCHED && B->dirty) {
