@@ -260,14 +260,14 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
     __syncthreads();  // a block may go on to another unit, which reuses sLL
 }
 
-// Row b of the partial sums covers the tiles b, b + blocks, b + 2*blocks, ...: a fixed function
+// Row b < rows of the partial sums covers the tiles b, b + rows, b + 2*rows, ...: a fixed function
 // of (N, blocks), whoever runs it, so every launch form (one graph, a batch of instances)
 // produces bitwise the same partial sums; blocks running at the same time read neighbouring
-// tiles.
+// tiles.  Further rows are zero.
 __device__ __forceinline__ void gmm_accumulate_unit(const float *__restrict__ X, const GMM_DIMS &d,
                                                     const double *__restrict__ model,
-                                                    double *__restrict__ partials, int b, GmmShared &sh) {
-    const long long t0 = b, t1 = ((long long)d.N + TILE - 1) / TILE, ts = d.blocks;
+                                                    double *__restrict__ partials, int b, int rows, GmmShared &sh) {
+    const long long t1 = ((long long)d.N + TILE - 1) / TILE, ts = rows, t0 = b < rows ? b : t1;
     double *row = partials + (long long)b * ptk_gmm_partial_stride(&d);
     switch (ptk_gmm_dpad(&d) >> 2) {
         case 1: gmm_accumulate_tiles<1>(X, d, model, row, t0, t1, ts, sh); break;

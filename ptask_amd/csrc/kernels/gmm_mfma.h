@@ -2,8 +2,9 @@
 // operand in registers.
 //
 //   GmmAccumulateMfma(const float* X, GMM_DIMS d, const double* model, double* partials)
-//     Same arguments, partial-row format and tile-to-row assignment as GmmAccumulate
-//     (gmm_body.h), so GmmFinalize and every caller are unchanged; only the rounding differs.
+//     Same arguments and partial-row format as GmmAccumulate (gmm_body.h), so GmmFinalize and every
+//     caller are unchanged; only the rounding differs, and the tiles go to the first
+//     GMM_MFMA_ROWS rows.
 //
 // A wave works alone on groups of 16 points, with coordinates centred on g (the mean of the
 // component means, one per-dimension vector per launch: x' = x - g, c'_k = mu_k - g):
@@ -30,8 +31,9 @@
 //
 // Bound: the matrix cores (8 N D K flops per step; 32 cycles of a SIMD per product).  Two waves per
 // SIMD (at most 256 registers) cover each other's log-sum-exp, about a quarter of the products'
-// issue time at D = 32, K = 64.  Measured there with N = 2M, 768 blocks: 328 us per launch, the matrix
-// cores busy 66% of the time; 612 us when tiles of coordinates and responsibilities passed through
+// issue time at D = 32, K = 64.  Measured there with N = 2M, 768 blocks: 300 us per launch (322 with
+// the tiles on all 768 rows, 309 without the log-sum-exp's priority), the matrix cores busy 70% of the
+// time; 612 us when tiles of coordinates and responsibilities passed through
 // LDS between the products (four barriers a tile, an LDS read per operand).  N = 50,001, D = 16, K = 24
 // (one tile per block): 13.5 us, 27.8 before, when every block first built the operand in LDS.
 #pragma once
@@ -42,6 +44,10 @@ typedef float gmm_f4 __attribute__((ext_vector_type(4)));
 
 #define GMM_MFMA_IV_LIMIT 1.0e3f
 #define GMM_GROUP 16  // points per wave and product
+// Partial rows that receive tiles; further ones are zero.  512 blocks are resident at once (two on each
+// of 256 CUs): of 768 the last 256 would have a CU each to themselves, where one wave per SIMD does not
+// cover its own log-sum-exp.
+#define GMM_MFMA_ROWS 512
 // doubles per component row of the block's moment sums (2 W moments): the four rows a wave's store
 // touches then start 32 banks apart
 #define GMM_ACC_STRIDE(W) (2 * (W) + 4)
@@ -115,6 +121,10 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
             }
         }
         if (__any(big)) return false;
+        if (t0 >= t1) {  // a row without a tile
+            for (int i = tid; i < K + 2 * K * D + 1; i += 256) row[i] = 0;
+            return true;
+        }
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
 #pragma unroll
@@ -265,6 +275,8 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
                 for (int kt = 0; kt < KT; ++kt)
                     e[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[i], b1[kt][i], e[kt], 0, 0, 0);
             // ---- log-sum-exp of point 4 l4 + r over the row's lanes; responsibilities into e
+            // (ahead of the SIMD's other wave, whose products fill the matrix core meanwhile)
+            __builtin_amdgcn_s_setprio(1);
             float mx[4], sum[4], lse[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -308,6 +320,7 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
                     x2[j][r] = x1[j][r] * x1[j][r];
                 }
             loadM(pn);
+            __builtin_amdgcn_s_setprio(0);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -398,7 +411,7 @@ __device__ __forceinline__ bool gmm_mfma_comps(const float *__restrict__ X, cons
 __device__ __forceinline__ void gmm_mfma_unit(const float *__restrict__ X, const GMM_DIMS &d,
                                               const double *__restrict__ model, double *__restrict__ partials,
                                               int b, GmmMfmaShared &sh) {
-    const long long t0 = b, t1 = ((long long)d.N + TILE - 1) / TILE, ts = d.blocks;
+    const long long t1 = ((long long)d.N + TILE - 1) / TILE, ts = min(d.blocks, GMM_MFMA_ROWS), t0 = b < ts ? b : t1;
     double *row = partials + (long long)b * ptk_gmm_partial_stride(&d);
     bool done;
     switch ((d.D + 7) >> 3) {
@@ -407,5 +420,5 @@ __device__ __forceinline__ void gmm_mfma_unit(const float *__restrict__ X, const
         case 3: done = gmm_mfma_comps<3>(X, d, model, row, t0, t1, ts, sh); break;
         default: done = gmm_mfma_comps<4>(X, d, model, row, t0, t1, ts, sh); break;
     }
-    if (!done) gmm_accumulate_unit(X, d, model, partials, b, sh.u.valu);
+    if (!done) gmm_accumulate_unit(X, d, model, partials, b, (int)ts, sh.u.valu);
 }
