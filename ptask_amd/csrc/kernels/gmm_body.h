@@ -49,6 +49,7 @@ struct GmmShared {
     float sMax[2][TILE];
     float sSum[2][TILE];
     double sLL[4];
+    int sNz[4];  // per wave of the E-phase: responsibilities that are not 0 (reps == 1)
 };
 
 // Coordinates of tile t (zero for padding points and dimensions, nothing for t >= t1) into this
@@ -167,7 +168,17 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         __syncthreads();
         const float tmp = mx + __logf(sh.sSum[0][ep] + sh.sSum[1][ep]);
         const bool valid = ep < np;
-        for (int k = k0; k < k1; ++k) sR[ep * RS + k] = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
+        if (reps == 1) {
+            int nz = 0;
+            for (int k = k0; k < k1; ++k) {
+                const float r = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
+                sR[ep * RS + k] = r;
+                nz += __popcll(__ballot(r != 0.f));
+            }
+            if (lane == 0) sh.sNz[wv] = nz;
+        } else {
+            for (int k = k0; k < k1; ++k) sR[ep * RS + k] = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
+        }
         if (valid && eh == 0) ll += (double)tmp;
         __syncthreads();
 
@@ -195,16 +206,26 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
             }
         };
         if (reps == 1) {  // the common large-K case keeps a unit-stride loop
-            // four points' responsibilities at a time; a point none of whose components here has any
-            // adds zeros and is passed over: before the variances have settled most are 0 in all but
-            // one component (2M points, D = 32, K = 64, the first step: 1,180 -> 830 us)
-            for (int p = 0; p < np; p += 4) {
-                float r[4];
+            // Before the variances have settled, and where components lie far apart, nearly every point
+            // has a responsibility in one component and 0 in the others.  In such a tile (five for four
+            // points, or fewer) a point none of whose components here has any adds zeros and is passed
+            // over; in any other tile the test of each point would cost more than it saves.  2M points,
+            // D = 32, K = 64, us per launch of GmmAccumulate with no test, this test, a test in every
+            // tile: one component a point 1,017, 887, 872; all overlapping 1,017, 1,007, 1,209 (and of
+            // GmmAccumulateMfma, which runs this body where its own E-step is not safe: 845, 745, 729
+            // and 842, 851, 981).
+            const int nz = __builtin_amdgcn_readfirstlane(sh.sNz[0] + sh.sNz[1] + sh.sNz[2] + sh.sNz[3]);
+            if (nz <= np + np / 4) {
+                for (int p = 0; p < np; p += 4) {
+                    float r[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) r[u] = fabsf(sR[(p + u) * RS + mk[0]]) + fabsf(sR[(p + u) * RS + mk[1]]);
+                    for (int u = 0; u < 4; ++u) r[u] = fabsf(sR[(p + u) * RS + mk[0]]) + fabsf(sR[(p + u) * RS + mk[1]]);
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (__any(r[u] != 0.f)) point(p + u);
+                    for (int u = 0; u < 4; ++u)
+                        if (__any(r[u] != 0.f)) point(p + u);
+                }
+            } else {
+                for (int p = 0; p < np; ++p) point(p);
             }
         } else {
             for (int p = grp; p < np; p += reps) point(p);
