@@ -353,6 +353,12 @@ __device__ inline void gb_partition_starts(const PTK_GB_SCRATCH &S, GbPartLds &L
 // u / 4), for inputs of so few chunks that most CUs would have none.  A quarter's block counts the
 // chunk's earlier quarters itself (three loads of keys at most), so no other pass changes.  500,000 rows
 // over 65536 keys: 31 chunks 27.7 us, 123 quarters 12.5 us.
+// BITS: how a step's rows find their peers of the same bucket: 8: through LDS words (up to 256 buckets),
+// otherwise with a ballot per bit of the bucket number.  In few buckets many lanes meet in one word, which
+// takes them one at a time, so up to 16 buckets have ballots.  Whole groupby, us, through words -> 2 ballots
+// (up to 4 buckets) or 4 (up to 16), rows with Zipf keys: 3.6M over 1001 keys 91.3 -> 86.5, over 2001 82.8 ->
+// 80.0, over 4001 79.0 -> 76.8; 8M over 1001 117.9 -> 110.3, over 2001 110.2 -> 107.3, over 4001 105.3 ->
+// 103.9.  Six ballots for 24 to 64 buckets gave 1 us at 3.3M rows and cost 2 at 8M.
 // blockDim.x == PTK_GB_PART_THREADS; begins and ends with a barrier.
 template <int BITS, bool QUARTERS>
 __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
@@ -362,7 +368,7 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
     int q = 0;
     if (QUARTERS) q = (int)(c % GB_PART_SUBS), c /= GB_PART_SUBS, cend = S.chunks;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    auto wcnt = [&](int v, unsigned b) -> unsigned short & { return BITS == 8 ? L.u.n.wcnt[v][b] : L.u.wcnt[v][b]; };
+    auto wcnt = [&](int v, unsigned b) -> unsigned short & { return BITS <= 8 ? L.u.n.wcnt[v][b] : L.u.wcnt[v][b]; };
     __syncthreads();
     for (int b = tid; b < NB; b += PTK_GB_PART_THREADS) L.bst[b] = S.btot[b];
     gb_lds_exscan(L.bst, NB, L.red);  // bucket starts
@@ -406,7 +412,7 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
             const long long row0 = c * PTK_GB_CHUNK + (long long)q * PTK_GB_SUB;
             const long long wr0 = row0 + (long long)w * (PTK_GB_SUB / GB_PART_WAVES);
             const int nin = wr0 >= n ? 0 : (n - wr0 < 64 * GB_PART_ROWS ? (int)(n - wr0) : 64 * GB_PART_ROWS);
-            if (BITS == 8) {
+            if (BITS == 8) {  // the counts and the words
                 for (int i = tid; i < (int)sizeof(L.u.n) / 16; i += PTK_GB_PART_THREADS) ((uint4 *)&L.u.n)[i] = make_uint4(0, 0, 0, 0);
             } else {
                 for (int v = 0; v < GB_PART_WAVES; ++v)
@@ -496,7 +502,9 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
 __device__ inline void gb_partition_chunks(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
                                            int numKeys, long long c, long long cend, long long step,
                                            const PTK_GB_SCRATCH &S, GbPartLds &L) {
-    if (S.buckets <= 256) gb_partition_chunks_t<8, false>(keys, vals, n, numKeys, c, cend, step, S, L);
+    if (S.buckets <= 4) gb_partition_chunks_t<2, false>(keys, vals, n, numKeys, c, cend, step, S, L);
+    else if (S.buckets <= 16) gb_partition_chunks_t<4, false>(keys, vals, n, numKeys, c, cend, step, S, L);
+    else if (S.buckets <= 256) gb_partition_chunks_t<8, false>(keys, vals, n, numKeys, c, cend, step, S, L);
     else gb_partition_chunks_t<11, false>(keys, vals, n, numKeys, c, cend, step, S, L);
 }
 
@@ -504,7 +512,9 @@ __device__ inline void gb_partition_chunks(const int *__restrict__ keys, const i
 __device__ inline void gb_partition_quarters(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
                                              int numKeys, long long u, long long step, const PTK_GB_SCRATCH &S,
                                              GbPartLds &L) {
-    if (S.buckets <= 256) gb_partition_chunks_t<8, true>(keys, vals, n, numKeys, u, 0, step, S, L);
+    if (S.buckets <= 4) gb_partition_chunks_t<2, true>(keys, vals, n, numKeys, u, 0, step, S, L);
+    else if (S.buckets <= 16) gb_partition_chunks_t<4, true>(keys, vals, n, numKeys, u, 0, step, S, L);
+    else if (S.buckets <= 256) gb_partition_chunks_t<8, true>(keys, vals, n, numKeys, u, 0, step, S, L);
     else gb_partition_chunks_t<11, true>(keys, vals, n, numKeys, u, 0, step, S, L);
 }
 
