@@ -328,7 +328,7 @@ BatchGmmAccumulate(const int2 *__restrict__ units, const int *__restrict__ count
     for (int u = blockIdx.x; u < n; u += gridDim.x) {
         const int2 w = units[u];
         const PTK_GMM_INST &I = insts[w.x];
-        gmm_accumulate_unit(I.X, I.d, I.model, I.partials, w.y, I.d.blocks, sh);
+        gmm_accumulate_unit<false>(I.X, I.d, I.model, I.partials, w.y, I.d.blocks, sh);
     }
 }
 

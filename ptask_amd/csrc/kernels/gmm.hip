@@ -13,7 +13,7 @@ GmmAccumulate(const float *__restrict__ X, GMM_DIMS d, const double *__restrict_
               double *__restrict__ partials) {
     __shared__ __align__(16) GmmShared sh;
     if (!gmm_dims_ok(d) || blockDim.x != 256 || (int)gridDim.x != d.blocks) return;
-    gmm_accumulate_unit(X, d, model, partials, (int)blockIdx.x, d.blocks, sh);
+    gmm_accumulate_unit<false>(X, d, model, partials, (int)blockIdx.x, d.blocks, sh);
 }
 
 extern "C" __global__ void __launch_bounds__(256, 2)

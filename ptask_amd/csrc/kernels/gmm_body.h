@@ -25,6 +25,9 @@
 //   M-phase: thread t owns (component, 4 dimensions) jobs t and t + 256 and walks the tile's
 //     points, reading the responsibility and a float4 of coordinates from LDS.
 // Tile sums are binary32 (128 points); the per-block running sums are binary64.
+//
+// GmmAccumulateMfma runs the same body where its own E-step is not safe (gmm_mfma.h), with the M-phase
+// on the matrix cores in binary64 (gmm_accumulate_tiles, MATRIX).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -71,7 +74,18 @@ __device__ __forceinline__ void gmm_fetch_tile(const float *__restrict__ X, cons
 // NC = float4 chunks per point (Dp / 4), a compile-time constant so that the chunk loops unroll
 // without guards and a component's table row arrives in one batch of scalar loads.
 // Tiles t0, t0 + tstep, ... (< t1) of the points into one row of partial sums.
-template <int NC>
+// MATRIX (K * NC > 128): the M-phase as one product R^T (K x 128) . [x' | x'^2] (128 x 2 Dp) per tile on
+// v_mfma_f64_16x16x4f64, x' = x - (the first component's mean), converted at the end to moments about the
+// table centres.  A wave has up to two pairs (16 components x 16 dimensions) of tiles, x' and x'^2, which
+// share both operands' loads.  Binary64 throughout, from exact differences: the conversion cancels by
+// c'^2 iv (1e4 where components lie a hundred deviations apart), which binary32 sums do not survive (a
+// relative error of 2e-5 in the variances there; 7e-8 in binary64 as about the table centres, all of it the
+// responsibilities').  Bound by the vector units' distances; the matrix cores take 230 us of the 706.
+// Per launch of GmmAccumulateMfma, us, against the jobs' vector loop with and without its test of each
+// point's responsibilities, and the 16x16x4 binary32 products of R and X: 2M points, D = 32, K = 64 where
+// all overlap 710 (840, 980, 967); the same where a point has one component 706 (845, 730, 967); 500,000 on 245
+// blocks of 16 tiles, D = 20, K = 64 238 (-, 450, 279); 300,000, D = 16, K = 48 68 (112, 134, 135).
+template <int NC, bool MATRIX>
 __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X, const GMM_DIMS &d,
                                                      const double *__restrict__ model,
                                                      double *__restrict__ row, long long t0,
@@ -115,6 +129,19 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
     }
     double ll = 0;
 
+    // MATRIX: pair i of the wave is components 16 kt[i] .., dimensions 16 dt ..; lane (l4, l16) supplies
+    // A[component l16][point l4] and B[point l4][dimension l16] and holds rows l4 + 4 r of column l16
+    typedef double gmm_d4 __attribute__((ext_vector_type(4)));
+    constexpr int DT = (4 * NC + 15) / 16;  // 1 or 2: the pairs wv and wv + 4 have the same dt
+    const int l16 = lane & 15, l4 = lane >> 4, pairs = ((K + 15) >> 4) * DT, dt = wv % DT;
+    const int mm = dt * 16 + l16;  // the lane's dimension; a column past D is never stored
+    const int kt[2] = {wv / DT, (wv + 4) / DT};
+    const double g = (double)tab[mm < D ? mm : D - 1];
+    gmm_d4 m1[2], m2[2];
+    double dw = 0;  // component `lane`, points 32 wv .. of the tiles
+#pragma unroll
+    for (int i = 0; i < 2; ++i) m1[i] = m2[i] = gmm_d4{0, 0, 0, 0};
+
     // The next tile's coordinates are loaded into registers while the current tile computes
     // (2 NC values per thread: TILE x Dp / 256), so the global-memory latency stays hidden.
     float pf[2 * NC];
@@ -140,7 +167,9 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
             x[4 * c + 2] = v.z;
             x[4 * c + 3] = v.w;
         }
+        if (MATRIX) __builtin_amdgcn_s_setprio(1);  // the other block's products fill the matrix cores
         float mx = -INFINITY;
+#pragma unroll 2
         for (int k = k0; k < k1; ++k) {
             const float *__restrict__ tk = tab + 2 * k * Dp;
             float s0 = 0.f, s1 = 0.f;
@@ -163,12 +192,13 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         __syncthreads();
         mx = fmaxf(sh.sMax[0][ep], sh.sMax[1][ep]);
         float sum = 0.f;
+#pragma unroll 8
         for (int k = k0; k < k1; ++k) sum += __expf(sR[ep * RS + k] - mx);
         sh.sSum[eh][ep] = sum;
         __syncthreads();
         const float tmp = mx + __logf(sh.sSum[0][ep] + sh.sSum[1][ep]);
         const bool valid = ep < np;
-        if (reps == 1) {
+        if (!MATRIX && reps == 1) {
             int nz = 0;
             for (int k = k0; k < k1; ++k) {
                 const float r = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
@@ -177,10 +207,39 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
             }
             if (lane == 0) sh.sNz[wv] = nz;
         } else {
+#pragma unroll 8
             for (int k = k0; k < k1; ++k) sR[ep * RS + k] = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
         }
         if (valid && eh == 0) ll += (double)tmp;
         __syncthreads();
+
+        // ---- M-phase on the matrix cores
+        if (MATRIX) {
+            __builtin_amdgcn_s_setprio(0);
+            double w[4] = {0, 0, 0, 0};
+#pragma unroll 2
+            for (int p = 32 * wv; p < 32 * wv + 32; p += 4)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[u] += (double)sR[(p + u) * RS + lane];
+            dw += (w[0] + w[1]) + (w[2] + w[3]);
+            if (wv < pairs) {
+#pragma unroll 4
+                for (int s = 0; s < TILE / 4; ++s) {  // a point past the last has responsibility 0
+                    const int p = 4 * s + l4;
+                    const double xp = (double)sX[p * XS + mm] - g;
+                    const double a = (double)sR[p * RS + 16 * kt[0] + l16];
+                    m1[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, xp, m1[0], 0, 0, 0);
+                    m2[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, xp * xp, m2[0], 0, 0, 0);
+                    if (wv + 4 < pairs) {
+                        const double b = (double)sR[p * RS + 16 * kt[1] + l16];
+                        m1[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, xp, m1[1], 0, 0, 0);
+                        m2[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, xp * xp, m2[1], 0, 0, 0);
+                    }
+                }
+            }
+            __syncthreads();
+            continue;
+        }
 
         // ---- M-phase: tile sums for jobs (mk, mc)
         float w[2], su[2][4], suu[2][4];
@@ -210,10 +269,8 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
             // has a responsibility in one component and 0 in the others.  In such a tile (five for four
             // points, or fewer) a point none of whose components here has any adds zeros and is passed
             // over; in any other tile the test of each point would cost more than it saves.  2M points,
-            // D = 32, K = 64, us per launch of GmmAccumulate with no test, this test, a test in every
-            // tile: one component a point 1,017, 887, 872; all overlapping 1,017, 1,007, 1,209 (and of
-            // GmmAccumulateMfma, which runs this body where its own E-step is not safe: 845, 745, 729
-            // and 842, 851, 981).
+            // D = 32, K = 64, us per launch of GmmAccumulate: 861 where a point has one component, 994
+            // where all overlap (1,209 with the test in every tile; 1,017 either way with none).
             const int nz = __builtin_amdgcn_readfirstlane(sh.sNz[0] + sh.sNz[1] + sh.sNz[2] + sh.sNz[3]);
             if (nz <= np + np / 4) {
                 for (int p = 0; p < np; p += 4) {
@@ -268,9 +325,27 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         __syncthreads();
     }
     // the row of partial sums
+    if (MATRIX) {
+        double *sW = (double *)sR;  // [4][KMAX]
+        sW[wv * KMAX + lane] = dw;
+        __syncthreads();
+        auto weight = [&](int k) { return sW[k] + sW[KMAX + k] + sW[2 * KMAX + k] + sW[3 * KMAX + k]; };
+        if (tid < K) row[tid] = weight(tid);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = 16 * kt[i] + l4 + 4 * r;
+                if (wv + 4 * i < pairs && k < K && mm < D) {
+                    const double wk = weight(k), c = (double)tab[2 * k * Dp + mm] - g;
+                    row[K + k * D + mm] = m1[i][r] - c * wk;
+                    row[K + K * D + k * D + mm] = m2[i][r] - 2.0 * c * m1[i][r] + c * c * wk;
+                }
+            }
+    }
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        if (!mv[q]) continue;
+        if (MATRIX || !mv[q]) continue;
         const int k = mk[q];
         if (mc[q] == 0) row[k] = aw[q];
 #pragma unroll
@@ -295,20 +370,33 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
 // of (N, blocks), whoever runs it, so every launch form (one graph, a batch of instances)
 // produces bitwise the same partial sums; blocks running at the same time read neighbouring
 // tiles.  Further rows are zero.
+template <bool MATRIX>
 __device__ __forceinline__ void gmm_accumulate_unit(const float *__restrict__ X, const GMM_DIMS &d,
                                                     const double *__restrict__ model,
                                                     double *__restrict__ partials, int b, int rows, GmmShared &sh) {
     const long long t1 = ((long long)d.N + TILE - 1) / TILE, ts = rows, t0 = b < rows ? b : t1;
     double *row = partials + (long long)b * ptk_gmm_partial_stride(&d);
-    switch (ptk_gmm_dpad(&d) >> 2) {
-        case 1: gmm_accumulate_tiles<1>(X, d, model, row, t0, t1, ts, sh); break;
-        case 2: gmm_accumulate_tiles<2>(X, d, model, row, t0, t1, ts, sh); break;
-        case 3: gmm_accumulate_tiles<3>(X, d, model, row, t0, t1, ts, sh); break;
-        case 4: gmm_accumulate_tiles<4>(X, d, model, row, t0, t1, ts, sh); break;
-        case 5: gmm_accumulate_tiles<5>(X, d, model, row, t0, t1, ts, sh); break;
-        case 6: gmm_accumulate_tiles<6>(X, d, model, row, t0, t1, ts, sh); break;
-        case 7: gmm_accumulate_tiles<7>(X, d, model, row, t0, t1, ts, sh); break;
-        default: gmm_accumulate_tiles<8>(X, d, model, row, t0, t1, ts, sh); break;
+    const int nc = ptk_gmm_dpad(&d) >> 2;
+    if (MATRIX && d.K * nc > 128) {  // so nc >= 3
+        switch (nc) {
+            case 3: gmm_accumulate_tiles<3, true>(X, d, model, row, t0, t1, ts, sh); break;
+            case 4: gmm_accumulate_tiles<4, true>(X, d, model, row, t0, t1, ts, sh); break;
+            case 5: gmm_accumulate_tiles<5, true>(X, d, model, row, t0, t1, ts, sh); break;
+            case 6: gmm_accumulate_tiles<6, true>(X, d, model, row, t0, t1, ts, sh); break;
+            case 7: gmm_accumulate_tiles<7, true>(X, d, model, row, t0, t1, ts, sh); break;
+            default: gmm_accumulate_tiles<8, true>(X, d, model, row, t0, t1, ts, sh); break;
+        }
+        return;
+    }
+    switch (nc) {
+        case 1: gmm_accumulate_tiles<1, false>(X, d, model, row, t0, t1, ts, sh); break;
+        case 2: gmm_accumulate_tiles<2, false>(X, d, model, row, t0, t1, ts, sh); break;
+        case 3: gmm_accumulate_tiles<3, false>(X, d, model, row, t0, t1, ts, sh); break;
+        case 4: gmm_accumulate_tiles<4, false>(X, d, model, row, t0, t1, ts, sh); break;
+        case 5: gmm_accumulate_tiles<5, false>(X, d, model, row, t0, t1, ts, sh); break;
+        case 6: gmm_accumulate_tiles<6, false>(X, d, model, row, t0, t1, ts, sh); break;
+        case 7: gmm_accumulate_tiles<7, false>(X, d, model, row, t0, t1, ts, sh); break;
+        default: gmm_accumulate_tiles<8, false>(X, d, model, row, t0, t1, ts, sh); break;
     }
 }
 

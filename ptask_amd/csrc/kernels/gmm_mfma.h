@@ -22,7 +22,7 @@
 //
 // The expansion in the E-step cancels (|x'|^2 iv against the distance); it runs only while every
 // reciprocal variance is at most GMM_MFMA_IV_LIMIT.  Otherwise (the first EM step, var = 1e-10) the
-// block runs GmmAccumulate's body.
+// block runs GmmAccumulate's body, its M-phase on the matrix cores in binary64.
 //
 // Sums are binary32 over at most 128 points of one wave (in MFMA order), then binary64 (LDS for the
 // block, or registers where the moments are few), converted once per block to moments about the
@@ -420,5 +420,5 @@ __device__ __forceinline__ void gmm_mfma_unit(const float *__restrict__ X, const
         case 3: done = gmm_mfma_comps<3>(X, d, model, row, t0, t1, ts, sh); break;
         default: done = gmm_mfma_comps<4>(X, d, model, row, t0, t1, ts, sh); break;
     }
-    if (!done) gmm_accumulate_unit(X, d, model, partials, b, (int)ts, sh.u.valu);
+    if (!done) gmm_accumulate_unit<true>(X, d, model, partials, b, (int)ts, sh.u.valu);
 }
