@@ -102,7 +102,8 @@ unsigned long long ptk_batch_footprint(int kind, long long a, int b_, int c, int
 
 /* One iteration: admit queued instances in submission order while they fit (at most max_admit,
  * < 0 = no limit), run one step of every active instance, retire completed ones.  *active and
- * *completed (either may be NULL) receive the counts after the iteration. */
+ * *completed (either may be NULL) receive the counts after the iteration.  When the admission
+ * itself fails, none of the call's instances is admitted: all are queued as before. */
 int ptk_batch_tick(ptk_batch *b, int max_admit, int *active, int *completed);
 /* As ptk_batch_tick, but runs up to max_iters iterations back to back without waiting between
  * them: as many as every resident instance still needs before the first of them completes (one

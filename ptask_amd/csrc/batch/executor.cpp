@@ -403,6 +403,17 @@ int Admit(ptk_batch *B, Inst &in) {
     return PTK_BATCH_OK;
 }
 
+// Takes back what Admit gave an instance, whether or not it was given all of it.  What is on the stream for
+// it still writes to its part of the arena, before anything a later owner puts there.
+void Unadmit(ptk_batch *B, Inst &in) {
+    std::vector<int> &slots = in.kind == PTK_INST_FDTD ? B->freeFdtd : in.kind == PTK_INST_GROUPBY ? B->freeGb : B->freeGmm;
+    if (in.slot >= 0) slots.push_back(in.slot);
+    in.slot = -1;
+    B->arena.Free(in.off, in.bytes);
+    in.state = PTK_STATE_QUEUED;
+    in.tAdmit = -1;
+}
+
 // Work lists of the resident instances for the batched kernels.
 // Whole-step tiles own 62 x 6 columns (blocks of 64 x 8 threads overlapping by one cell);
 // three-step tiles own 58 x 10 (blocks of 64 x 16 threads overlapping by three cells).
@@ -959,25 +970,23 @@ int ptk_batch_submit_gmm(ptk_batch *B, int n, int d, int k, int steps, unsigned 
 int ptk_batch_run(ptk_batch *B, int max_admit, int max_iters, int *niters, int *nactive, int *ncompleted) {
     if (!B || max_iters < 1) return Fail(PTK_BATCH_EINVAL, "bad argument");
     // admission: in submission order while the footprint fits
-    int admitted = 0;
-    size_t qi = 0;
-    std::vector<int> fdtd;
-    while (qi < B->queue.size() && (max_admit < 0 || admitted < max_admit)) {
-        Inst &in = B->insts[(size_t)B->queue[qi]];
+    std::vector<int> placed, fdtd;  // in queue order; the FDTD instances among them
+    int r = PTK_BATCH_OK;
+    while (placed.size() < B->queue.size() && (max_admit < 0 || (int)placed.size() < max_admit)) {
+        Inst &in = B->insts[(size_t)B->queue[placed.size()]];
         if (!B->arena.Alloc(in.bytes, &in.off)) break;
-        if (int r = Admit(B, in)) {
-            B->arena.Free(in.off, in.bytes);
-            InitFdtd(B, fdtd);
-            return r;
-        }
+        placed.push_back(in.id);
         if (in.kind == PTK_INST_FDTD) fdtd.push_back(in.id);
-        B->active.push_back(in.id);
-        ++admitted;
-        ++qi;
+        if ((r = Admit(B, in))) break;
     }
-    if (int r = InitFdtd(B, fdtd)) return r;
-    B->queue.erase(B->queue.begin(), B->queue.begin() + (long)qi);
-    if (admitted) B->dirty = true;
+    if (!r) r = InitFdtd(B, fdtd);
+    if (r) {  // none of them is admitted: all are queued as before the call
+        for (size_t i = placed.size(); i-- > 0;) Unadmit(B, B->insts[(size_t)placed[i]]);
+        return r;
+    }
+    B->active.insert(B->active.end(), placed.begin(), placed.end());
+    B->queue.erase(B->queue.begin(), B->queue.begin() + (long)placed.size());
+    if (!placed.empty()) B->dirty = true;
     if (!B->active.empty() && B->mode == PTK_BATCH_BATCHED && B->dirty) {
         if (int r = BuildLists(B)) return r;
         B->dirty = false;
