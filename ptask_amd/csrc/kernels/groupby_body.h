@@ -155,10 +155,12 @@ __device__ __forceinline__ unsigned long long gb_match_lds(unsigned d, bool use,
 // time).  Copies start on different banks (an odd stride); more than GB_HIST_COPIED buckets have one copy.
 #define GB_HIST_COPIED 256
 #define GB_HIST_COPIES 8
+#define GB_HIST_COPY_WORDS (GB_HIST_COPIES * (GB_HIST_COPIED + 1))
 struct GbHistLds {
     union {
         unsigned one[PTK_GB_MAX_BUCKETS];
         unsigned copy[GB_HIST_COPIES][GB_HIST_COPIED + 1];
+        unsigned words[GB_HIST_COPY_WORDS];  // all of copy
     } cnt;
     unsigned long long red[16];
 };
@@ -198,9 +200,11 @@ __device__ inline void gb_histogram_chunk(const int *__restrict__ keys, long lon
     const long long r0 = c * PTK_GB_CHUNK, nr = n - r0 < PTK_GB_CHUNK ? n - r0 : PTK_GB_CHUNK;
     const bool copied = NB <= GB_HIST_COPIED;
     unsigned *const mine = copied ? L.cnt.copy[tid % GB_HIST_COPIES] : L.cnt.one;
-    const int words = copied ? GB_HIST_COPIES * (GB_HIST_COPIED + 1) : NB;
     __syncthreads();
-    for (int b = tid; b < words; b += PTK_GB_HIST_THREADS) L.cnt.one[b] = 0;
+    if (copied)
+        for (int i = tid; i < GB_HIST_COPY_WORDS; i += PTK_GB_HIST_THREADS) L.cnt.words[i] = 0;
+    else
+        for (int b = tid; b < NB; b += PTK_GB_HIST_THREADS) L.cnt.one[b] = 0;
     int4 kv[GB_HIST_ROWS / 4];
     const int4 *k4 = (const int4 *)(keys + r0);  // r0 is a multiple of 4: 16-byte aligned
     unsigned inRange = GB_HIST_ROWS;
