@@ -286,7 +286,7 @@ __device__ inline void gb_bucketscan(const PTK_GB_SCRATCH &S, int b, unsigned *r
 #define GB_PART_SUBS (PTK_GB_CHUNK / PTK_GB_SUB)         // quarter chunks per chunk
 
 struct GbPartLds {
-    union {
+    union alignas(16) {  // n is cleared 16 bytes at a time
         unsigned short wcnt[GB_PART_WAVES][PTK_GB_MAX_BUCKETS];  // per wave and bucket: rows, then the wave's base
         struct {                                                  // up to 256 buckets
             unsigned short wcnt[GB_PART_WAVES][256];
@@ -302,6 +302,7 @@ struct GbPartLds {
     unsigned red[16];
     unsigned long long red64[16];
 };
+static_assert(sizeof(GbPartLds::u.n) % 16 == 0, "whole 16-byte words");
 
 // After the bucket scan, by one block of the partition launch: the bucket starts (S.bstart) and
 // the first tile of each bucket (S.tstart), which the later passes read.  Any blockDim.x (a
