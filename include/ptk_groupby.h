@@ -98,7 +98,8 @@ PTK_GB_FN long long ptk_gb_tiles_max(long long n, int numKeys) {
 }
 /* Blocks of a GroupbyPartition launch on `cus` compute units, two of which fit each: one per quarter
  * chunk while they run in two rounds at most, else up to one per chunk, and one more for the starts and
- * the tile table.  (A quarter takes 11 us, or 7 with a CU to itself: 3M rows 22 us against 28.) */
+ * the tile table.  (3M rows over 65536 keys: 24.9 us in quarters against 28.3 in chunks; 500,000: 11.7
+ * against 27.5.) */
 PTK_GB_FN unsigned int ptk_gb_part_grid(long long n, int cus) {
     const long long chunks = ptk_gb_chunks(n), most = 2ll * (cus > 0 ? cus : 1);
     const long long quarters = chunks * (PTK_GB_CHUNK / PTK_GB_SUB);

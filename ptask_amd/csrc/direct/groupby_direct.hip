@@ -55,7 +55,6 @@ int LaunchSmall(const int *keys, const int *vals, int n, int numKeys, long long 
 int Launch(const int *keys, const int *vals, int n, int numKeys, long long *table, void *scratch, long long *offsets,
            long long *groups, int *outKeys, int *outVals, hipStream_t stream) {
     if (n <= 4 * GB_SMALL_THREADS) return LaunchSmall<4>(keys, vals, n, numKeys, offsets, groups, outKeys, outVals, stream);
-    if (n <= 4 * GB_SMALL_THREADS) return LaunchSmall<4>(keys, vals, n, numKeys, offsets, groups, outKeys, outVals, stream);
     if (n <= GB_SMALL_ROWS) return LaunchSmall<GB_SMALL_RPT>(keys, vals, n, numKeys, offsets, groups, outKeys, outVals, stream);
     const unsigned chunks = (unsigned)ptk_gb_chunks(n), nb = (unsigned)ptk_gb_buckets(numKeys);
     const unsigned tiles = (unsigned)ptk_gb_tiles_max(n, numKeys);

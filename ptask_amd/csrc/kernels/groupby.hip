@@ -65,7 +65,7 @@ GroupbyPartition(const int *__restrict__ keys, const int *__restrict__ vals, int
         gb_partition_starts(S, L);
     }
     if (b >= G) return;
-    if (quarters) gb_partition_quarters(keys, vals, n, numKeys, gb_xcd_block(b, G), G, S, L);
+    if (quarters) gb_partition_quarter(keys, vals, n, numKeys, gb_xcd_block(b, G), S, L);
     else gb_partition_chunks(keys, vals, n, numKeys, gb_xcd_block(b, G), S.chunks, G, S, L);
 }
 

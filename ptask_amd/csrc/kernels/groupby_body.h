@@ -354,10 +354,10 @@ __device__ inline void gb_partition_starts(const PTK_GB_SCRATCH &S, GbPartLds &L
 // time: writes each row's low key byte and value to S.tlow / S.tval at bstart[bucket] + the
 // earlier chunks' rows of the bucket + the row's rank among the chunk's rows of the bucket (row
 // order).  The next quarter's rows are loaded while the current quarter's are written.
-// QUARTERS: the units c, c + step, ... below cend are quarter chunks (unit u: quarter u % 4 of chunk
-// u / 4), for inputs of so few chunks that most CUs would have none.  A quarter's block counts the
-// chunk's earlier quarters itself (three loads of keys at most), so no other pass changes.  500,000 rows
-// over 65536 keys: 31 chunks 27.7 us, 123 quarters 12.5 us.
+// QUARTER: one quarter chunk (unit c: quarter c % 4 of chunk c / 4), for inputs of so few chunks that
+// most CUs would have none.  A quarter's block counts the chunk's earlier quarters itself (three loads
+// of keys at most), so no other pass changes.  500,000 rows over 65536 keys: 31 chunks 27.7 us, 123
+// quarters 12.5 us.
 // BITS: how a step's rows find their peers of the same bucket: 8: through LDS words (up to 256 buckets),
 // otherwise with a ballot per bit of the bucket number.  In few buckets many lanes meet in one word, which
 // takes them one at a time, so up to 16 buckets have ballots.  Whole groupby, us, through words -> 2 ballots
@@ -365,13 +365,13 @@ __device__ inline void gb_partition_starts(const PTK_GB_SCRATCH &S, GbPartLds &L
 // 80.0, over 4001 79.0 -> 76.8; 8M over 1001 117.9 -> 110.3, over 2001 110.2 -> 107.3, over 4001 105.3 ->
 // 103.9.  Six ballots for 24 to 64 buckets gave 1 us at 3.3M rows and cost 2 at 8M.
 // blockDim.x == PTK_GB_PART_THREADS; begins and ends with a barrier.
-template <int BITS, bool QUARTERS>
+template <int BITS, bool QUARTER>
 __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
                                              int numKeys, long long c, long long cend, long long step,
                                              const PTK_GB_SCRATCH &S, GbPartLds &L) {
     const int NB = (int)S.buckets;
     int q = 0;
-    if (QUARTERS) q = (int)(c % GB_PART_SUBS), c /= GB_PART_SUBS, cend = S.chunks;
+    if (QUARTER) q = (int)(c % GB_PART_SUBS), c /= GB_PART_SUBS, cend = S.chunks;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     auto wcnt = [&](int v, unsigned b) -> unsigned short & { return BITS <= 8 ? L.u.n.wcnt[v][b] : L.u.wcnt[v][b]; };
     __syncthreads();
@@ -384,21 +384,11 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
         gb_load_rows<GB_PART_ROWS>(vals, wr0, n, vr);
     };
     if (c < cend) fetch(c * PTK_GB_CHUNK + (long long)q * PTK_GB_SUB);
-    // one quarter chunk per iteration: (c, q), q = 0..GB_PART_SUBS - 1, then c += step (QUARTERS: one, then
-    // step quarters on)
-    auto next = [&]() {
-        if (QUARTERS) {
-            const long long u = c * GB_PART_SUBS + q + step;
-            c = u / GB_PART_SUBS, q = (int)(u % GB_PART_SUBS);
-        } else {
-            q = q + 1 < GB_PART_SUBS ? q + 1 : 0;
-            c += q == 0 ? step : 0;
-        }
-    };
-    for (; c < cend; next()) {
-        if (QUARTERS || q == 0)
+    // one quarter chunk per iteration: (c, q), q = 0..GB_PART_SUBS - 1, then c += step
+    for (; c < cend; q = q + 1 < GB_PART_SUBS ? q + 1 : 0, c += q == 0 ? step : 0) {
+        if (QUARTER || q == 0)
             for (int b = tid; b < NB; b += PTK_GB_PART_THREADS) L.dest[b] = L.bst[b] + S.hist[c * NB + b];
-        if (QUARTERS && q > 0) {
+        if (QUARTER && q > 0) {
             __syncthreads();
             const long long r0 = c * PTK_GB_CHUNK, r1 = r0 + (long long)q * PTK_GB_SUB < n ? r0 + (long long)q * PTK_GB_SUB : n;
             for (long long r = r0 + tid; r < r1; r += 8 * PTK_GB_PART_THREADS) {
@@ -468,10 +458,7 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
             for (int s = 0; s < GB_PART_ROWS; ++s)
                 if (rk[s] < PTK_GB_SUB) L.u.stage[rk[s]] = make_int2(kr[s], vr[s]);  // every valid row (rk < PTK_GB_SUB)
             __syncthreads();
-            if (QUARTERS) {  // in flight while this quarter is written
-                const long long u = c * GB_PART_SUBS + q + step;
-                if (u < cend * GB_PART_SUBS) fetch(u * PTK_GB_SUB);
-            } else {
+            if (!QUARTER) {  // in flight while this quarter is written
                 if (q + 1 < GB_PART_SUBS) fetch(row0 + PTK_GB_SUB);
                 else if (c + step < cend) fetch((c + step) * PTK_GB_CHUNK);
             }
@@ -500,10 +487,11 @@ __device__ inline void gb_partition_chunks_t(const int *__restrict__ keys, const
             }
             __syncthreads();
         }
+        if (QUARTER) return;
     }
 }
 
-// The two bucket-number widths: up to 256 buckets (65536 keys) and up to PTK_GB_MAX_BUCKETS.
+// Chunks c, c + step, ... below cend.
 __device__ inline void gb_partition_chunks(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
                                            int numKeys, long long c, long long cend, long long step,
                                            const PTK_GB_SCRATCH &S, GbPartLds &L) {
@@ -513,14 +501,13 @@ __device__ inline void gb_partition_chunks(const int *__restrict__ keys, const i
     else gb_partition_chunks_t<11, false>(keys, vals, n, numKeys, c, cend, step, S, L);
 }
 
-// Quarter chunks u, u + step, ... of all of them.
-__device__ inline void gb_partition_quarters(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
-                                             int numKeys, long long u, long long step, const PTK_GB_SCRATCH &S,
-                                             GbPartLds &L) {
-    if (S.buckets <= 4) gb_partition_chunks_t<2, true>(keys, vals, n, numKeys, u, 0, step, S, L);
-    else if (S.buckets <= 16) gb_partition_chunks_t<4, true>(keys, vals, n, numKeys, u, 0, step, S, L);
-    else if (S.buckets <= 256) gb_partition_chunks_t<8, true>(keys, vals, n, numKeys, u, 0, step, S, L);
-    else gb_partition_chunks_t<11, true>(keys, vals, n, numKeys, u, 0, step, S, L);
+// Quarter chunk u.
+__device__ inline void gb_partition_quarter(const int *__restrict__ keys, const int *__restrict__ vals, long long n,
+                                            int numKeys, long long u, const PTK_GB_SCRATCH &S, GbPartLds &L) {
+    if (S.buckets <= 4) gb_partition_chunks_t<2, true>(keys, vals, n, numKeys, u, 0, 1, S, L);
+    else if (S.buckets <= 16) gb_partition_chunks_t<4, true>(keys, vals, n, numKeys, u, 0, 1, S, L);
+    else if (S.buckets <= 256) gb_partition_chunks_t<8, true>(keys, vals, n, numKeys, u, 0, 1, S, L);
+    else gb_partition_chunks_t<11, true>(keys, vals, n, numKeys, u, 0, 1, S, L);
 }
 
 // Tile t of the partitioned rows (t < S.tstart[NB]): its bucket and row range.
@@ -580,9 +567,9 @@ __device__ inline void gb_keycount_tile(const PTK_GB_SCRATCH &S, unsigned t, GbK
 #define GB_KS_PARTS (PTK_GB_KEYSCAN_THREADS / GB_KS_KEYS)    // threads per key in keyscan
 // Tiles whose counts a keyscan thread loads at once.  Sixteen leave the kernel under 64 registers, so
 // that two of its 1024-thread blocks fit a CU (the kernels ask for that): most buckets have a few tiles
-// and the launch lasts as long as its rounds of blocks.  Whole groupby, us, against forty tiles at once on
-// 110 registers: 1M rows over 262144 keys 77.5 (87.9), 500,000 over 65536 45.6 (48.4), 8M over 65536
-// 117.8 (118.5); and 8M over 16, whose one bucket has 1953 tiles, 222 (227).
+// and the launch lasts as long as its rounds of blocks.  Whole groupby of Zipf keys, us, with 16, 24 and 32:
+// 1M rows over 262144 keys 79.6, 91.7, 111.6; 500,000 over 65536 44.5, 47.8, 54.0; 8M over 65536 112.3, 118.6,
+// 122.0; and 8M over 16, whose one bucket has 1953 tiles, 141.0, 146.2, 147.5.
 #ifndef GB_KS_BATCH
 #define GB_KS_BATCH 16
 #endif
