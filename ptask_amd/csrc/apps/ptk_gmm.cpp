@@ -38,7 +38,7 @@ struct Options {
     std::string kernelFile, data, dump, mode = "looped", init;
     long long n = 100000;
     int d = 8, k = 8, steps = 10;
-    int blocks = 0;  // GmmAccumulate blocks; 0 = min(tiles, 768): three 128-point tiles per CU
+    int blocks = 0;  // accumulate blocks; 0 = min(tiles, 768) (GmmAccumulateMfma gives tiles to the first 512)
     int repeat = 1, warmup = 0;
     unsigned long long seed = 0x6a5d39;
     bool profile = false;

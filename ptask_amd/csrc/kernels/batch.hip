@@ -110,10 +110,10 @@ BatchFdtdStep(const int4 *__restrict__ tiles, const int *__restrict__ count, con
 // once.  A launch reads set (done & 1) and writes the other set three steps later, so one
 // BatchFdtdAdvance per launch keeps the set index right.  Same instance conditions as BatchFdtdStep.
 // count[5]: there are fewer tiles than virtual blocks.  Then a launch lasts as long as one segment's
-// planes, and column_tile forms them (fdtd_fused.h): 24 instances of edge 16..40, 29 us per launch
-// against 50 with overlapn_tile on equal runs.  With more tiles (2048 instances of edge 16..96)
-// HBM and the overlap's reuse in L2 count, as at 384^3, and overlapn_tile is the faster: 205 ms of
-// execution for 50 steps against 215.
+// planes, and column_tile forms them (fdtd_fused.h); with many more, HBM and the overlap's reuse in L2
+// count, as at 384^3, and overlapn_tile is the faster.  50 steps of n instances in all, ms, with
+// column_tile, overlapn_tile on the same schedule, and overlapn_tile on equal runs: 24 of edge 16 to 40 0.78,
+// 0.99, 1.20; 12 of 96 3.26, 3.56, 3.90; 500 of 16 to 96 56.7, 48.6, 51.2; 2048 of 16 to 96 251, 209, 227.
 template <class Tile>
 __device__ __forceinline__ void batch_steps3(const int4 *__restrict__ tiles, int G, const int *__restrict__ starts,
                                              const PTK_FDTD_INST *__restrict__ insts, Tile tile) {

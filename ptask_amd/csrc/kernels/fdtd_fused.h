@@ -626,15 +626,22 @@ __device__ inline void overlapn_tile(const Fields &F, const FDTD_PARAMS &p, int 
 //         B orders every access.
 // A step is formed only in the iterations that need it: with T = 3, owned planes [k0, k1) need H_s
 // from iteration 3(s - 1) on (counted from plane k0 - T) and E_s up to T - s iterations before the
-// last, so a slab of n planes takes n + 7 iterations and 3n + 9 step planes instead of 3n + 21: most
-// of the work of the short slabs that a small problem is cut into.
-// Measured: 64^3, three steps on 256 blocks: 22.0 us per launch against 41.9 (35.5 before the short
-// slabs and the skipped steps, 25.1 with the slabs alone).  At 384^3
-// it is the slower one, 890 us against 755: it computes a launch in 460 us when nothing is read or
-// written, so the blocks run at the pace of memory and drift apart, and neighbouring tiles then fetch
-// the three cells they share twice (FETCH_SIZE 2.12 GB against 1.67).  overlapn_tile's two barriers
-// and fuller planes keep the blocks in step.  So this body serves the launches with fewer tiles than
-// blocks (and the batched small instances), overlapn_tile the others.
+// last, so a slab of n planes takes 8 + 4 ceil((n - 1) / 4) iterations (the inner ones run in groups of
+// four) and 3n + 9 step planes or up to 9 more, instead of 3n + 21: most of the work of the short slabs that
+// a small problem is cut into.
+// Measured, us per three-step launch on 256 blocks, against overlapn_tile on the same slabs and on equal
+// runs of planes:
+//   48^3 14.6, 21.2, 20.1;  64^3 21.4, 28.8, 41.3;  96^3 25.2, 33.8, 46.6;  128^3 45.9, 58.6, 66.2;
+//   160^3 56.1, 72.4, 84.6;  192^3 129, 125, 135;  224^3 212, 219, 219;  248^3 234, 224, 284;
+//   256^3 317, 319, 320;  288^3 572, 573, 574;  320^3 917, 920, 921;  344^3 1128, 1135, 1135;
+//   200 x 200 x 800 537, 476, 701;  320 x 320 x 32 60.6, 74.1, 73.2.
+// So it is the faster while the fields of a launch lie in cache, and once they do not the two stay within
+// 5% of each other, either way, but for a few shapes (80 to 126 tiles of 340 to 730 MB, and 200 x 200 x 800)
+// that no line through tiles, planes or bytes separates.  With more tiles than blocks it is the slower,
+// 890 us against 755 at 384^3: it computes a launch in 460 us when nothing is read or written, so the blocks
+// run at the pace of memory and drift apart, and neighbouring tiles then fetch the three cells they share
+// twice (FETCH_SIZE 2.12 GB against 1.67).  overlapn_tile's two barriers and fuller planes keep the blocks
+// in step.  So this body serves the launches with fewer tiles than blocks, overlapn_tile the others.
 template <int T, int MAXR>
 struct ColumnLds {
     float e[T][2][2][MAXR + 1][64]; // Ex, Ez of E_0 .. E_{T-1}: row r's at [r]
