@@ -120,7 +120,7 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
                 s[i] += (double)b1[kt][i];
             }
         }
-        if (__any(big)) return false;
+        if (__builtin_expect(__any(big), 0)) return false;  // unlikely: the other body's code lies behind this one's
         if (t0 >= t1) {  // a row without a tile
             for (int i = tid; i < K + 2 * K * D + 1; i += 256) row[i] = 0;
             return true;
