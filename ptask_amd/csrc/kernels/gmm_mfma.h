@@ -98,8 +98,11 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const float *__restrict__ tab = (const float *)(model + ptk_gmm_table(&d));
 
-    // ---- per launch: the centre and the E-step operand of this lane's dimensions f0 .. f0 + NF - 1
-    const int f0 = l4 * NF;
+    // ---- per launch: the centre and the E-step operand of this lane's dimensions f0 .. f0 + NF - 1, those
+    // from l4 NF on.  Where these run past D the lane starts earlier, at dimensions of lanes before it, with
+    // zeros in the operand there: it then loads coordinates of its point only.  (One dimension is fewer
+    // than NF: the second of a lane's is none of the point's.)
+    const int f0 = D < NF ? 0 : min(l4 * NF, D - NF);
     float g[NF], b1[KT][NF], b2[KT][NF], ek[KT];
     bool big = false;
     {
@@ -111,10 +114,10 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
             const int k = kt * 16 + l16;
 #pragma unroll
             for (int i = 0; i < NF; ++i) {
-                const bool on = k < K && f0 + i < D;
+                const bool in = k < K && f0 + i < D, on = in && f0 + i >= l4 * NF;
                 const float *e = tab + 2 * (k < K ? k : 0) * Dp + (f0 + i < D ? f0 + i : 0);
                 const float mu = e[0], iv = e[Dp];
-                b1[kt][i] = on ? mu : 0.f;
+                b1[kt][i] = in ? mu : 0.f;
                 b2[kt][i] = on ? iv : 0.f;
                 if (on && !(iv <= GMM_MFMA_IV_LIMIT)) big = true;
                 s[i] += (double)b1[kt][i];
@@ -129,11 +132,12 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
         for (int i = 0; i < NF; ++i) {
 #pragma unroll
             for (int off = 1; off < 16; off <<= 1) s[i] += __shfl_xor(s[i], off, 64);
-            g[i] = (float)(s[i] / K);  // 0 for i past D
+            g[i] = (float)(s[i] / K);
         }
         if (wv == 0 && l16 == 0)
 #pragma unroll
-            for (int i = 0; i < NF; ++i) sh.g[f0 + i] = g[i];
+            for (int i = 0; i < NF; ++i)
+                if (f0 + i >= l4 * NF && f0 + i < D) sh.g[f0 + i] = g[i];
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
             const int k = kt * 16 + l16;
@@ -162,7 +166,7 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
     for (int j = 0; j < NS; ++j) {
         const int c = 16 * j + l16, m = c < W ? c : c - W;
         jd[j] = m < D ? m : D - 1;  // a column past D is never read back
-        gm[j] = sh.g[m];
+        gm[j] = sh.g[jd[j]];
     }
 
     gmm_f4 acc[KT][JT];
@@ -204,9 +208,8 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
 
     // Wave wv takes points [32 wv, 32 wv + 32) of each 128-point tile, as two groups: group n of the
     // wave is points 16 (n & 1) .. of tile t0 + (n >> 1) tstep.  A group's coordinates are loaded
-    // while the group before it computes, through a buffer that ends with the last point: what lies
-    // past it reads as 0 (such a point gets responsibility 0; a dimension past D is multiplied by 0
-    // or never read back), so a group is always the same loads, whatever D and its alignment.
+    // while the group before it computes, through a buffer that ends with the last point (what lies past it
+    // reads as 0), so a group is always the same loads, whatever D and its alignment.
     float xe[NF], xm[NS][4];
     auto base = [&](long long t, int q) { return t * TILE + 32 * wv + 16 * q; };
     auto group = [&](long long p0) {
@@ -255,6 +258,11 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
             const int np = (int)min((long long)GMM_GROUP, d.N - p0);  // valid points (<= 0: none)
             // ---- E-step
             float a1[NF], a2[NF];
+            // a point past the last, whose square may overflow, lies at the centre
+            if (__builtin_expect(D < NF || np < GMM_GROUP, 0)) {
+#pragma unroll
+                for (int i = 0; i < NF; ++i) xe[i] = f0 + i < D && l16 < np ? xe[i] : g[i];
+            }
 #pragma unroll
             for (int i = 0; i < NF; ++i) {
                 a1[i] = xe[i] - g[i];
@@ -311,6 +319,12 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
                 if (l16 < 4 && 4 * l4 + l16 < np) ll += (double)v;
             }
             // ---- M-step
+            if (__builtin_expect(np < GMM_GROUP, 0)) {
+#pragma unroll
+                for (int j = 0; j < NS; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) xm[j][r] = 4 * l4 + r < np ? xm[j][r] : gm[j];
+            }
             float x1[NS][4], x2[NS][4];
 #pragma unroll
             for (int j = 0; j < NS; ++j)
