@@ -74,7 +74,7 @@ __device__ __forceinline__ void gmm_fetch_tile(const float *__restrict__ X, cons
 // NC = float4 chunks per point (Dp / 4), a compile-time constant so that the chunk loops unroll
 // without guards and a component's table row arrives in one batch of scalar loads.
 // Tiles t0, t0 + tstep, ... (< t1) of the points into one row of partial sums.
-// MATRIX (K * NC > 128): the M-phase as one product R^T (K x 128) . [x' | x'^2] (128 x 2 Dp) per tile on
+// MATRIX (K * NC > 40): the M-phase as one product R^T (K x 128) . [x' | x'^2] (128 x 2 Dp) per tile on
 // v_mfma_f64_16x16x4f64, x' = x - (the first component's mean), converted at the end to moments about the
 // table centres.  A wave has up to two pairs (16 components x 16 dimensions) of tiles, x' and x'^2, which
 // share both operands' loads.  Binary64 throughout, from exact differences: the conversion cancels by
@@ -85,6 +85,9 @@ __device__ __forceinline__ void gmm_fetch_tile(const float *__restrict__ X, cons
 // point's responsibilities, and the 16x16x4 binary32 products of R and X: 2M points, D = 32, K = 64 where
 // all overlap 710 (840, 980, 967); the same where a point has one component 706 (845, 730, 967); 500,000 on 245
 // blocks of 16 tiles, D = 20, K = 64 238 (-, 450, 279); 300,000, D = 16, K = 48 68 (112, 134, 135).
+// Few components or dimensions leave the products' tiles empty and the jobs' threads full.  300,000 points,
+// products against jobs: 96 jobs (D = 16, K = 24) 52 and 72, 64 (32, 8) 46 and 48, 48 (16, 12) 37 and 41; 40
+// (8, 20) 42 and 39, 32 (32, 4) 41 and 33.
 template <int NC, bool MATRIX>
 __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X, const GMM_DIMS &d,
                                                      const double *__restrict__ model,
@@ -169,7 +172,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         }
         if (MATRIX) __builtin_amdgcn_s_setprio(1);  // the other block's products fill the matrix cores
         float mx = -INFINITY;
-#pragma unroll 2
+#pragma unroll(MATRIX || NC <= 2 ? 2 : 1)
         for (int k = k0; k < k1; ++k) {
             const float *__restrict__ tk = tab + 2 * k * Dp;
             float s0 = 0.f, s1 = 0.f;
@@ -192,7 +195,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         __syncthreads();
         mx = fmaxf(sh.sMax[0][ep], sh.sMax[1][ep]);
         float sum = 0.f;
-#pragma unroll 8
+#pragma unroll(MATRIX ? 8 : 2)
         for (int k = k0; k < k1; ++k) sum += __expf(sR[ep * RS + k] - mx);
         sh.sSum[eh][ep] = sum;
         __syncthreads();
@@ -207,7 +210,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
             }
             if (lane == 0) sh.sNz[wv] = nz;
         } else {
-#pragma unroll 8
+#pragma unroll(MATRIX ? 8 : 2)
             for (int k = k0; k < k1; ++k) sR[ep * RS + k] = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
         }
         if (valid && eh == 0) ll += (double)tmp;
@@ -299,7 +302,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         __syncthreads();
     }
 
-    if (reps > 1) {  // combine the groups' sums in group order (LDS of sR is free now)
+    if (!MATRIX && reps > 1) {  // combine the groups' sums in group order (LDS of sR is free now)
         double *acc = (double *)sR;
         if (mv[0] || tid < reps * jobs) {
             double *a = acc + (size_t)tid * 9;
@@ -377,8 +380,10 @@ __device__ __forceinline__ void gmm_accumulate_unit(const float *__restrict__ X,
     const long long t1 = ((long long)d.N + TILE - 1) / TILE, ts = rows, t0 = b < rows ? b : t1;
     double *row = partials + (long long)b * ptk_gmm_partial_stride(&d);
     const int nc = ptk_gmm_dpad(&d) >> 2;
-    if (MATRIX && d.K * nc > 128) {  // so nc >= 3
+    if (MATRIX && d.K * nc > 40) {
         switch (nc) {
+            case 1: gmm_accumulate_tiles<1, true>(X, d, model, row, t0, t1, ts, sh); break;
+            case 2: gmm_accumulate_tiles<2, true>(X, d, model, row, t0, t1, ts, sh); break;
             case 3: gmm_accumulate_tiles<3, true>(X, d, model, row, t0, t1, ts, sh); break;
             case 4: gmm_accumulate_tiles<4, true>(X, d, model, row, t0, t1, ts, sh); break;
             case 5: gmm_accumulate_tiles<5, true>(X, d, model, row, t0, t1, ts, sh); break;

@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("N,blocks", [(1, 1), (129, 2), (1500, 3), (3001, 24)])
-@pytest.mark.parametrize("D,K", [(9, 43), (12, 44), (13, 34), (16, 33), (17, 26), (20, 64), (28, 19), (32, 17), (32, 64)])
+@pytest.mark.parametrize("D,K", [(1, 41), (4, 64), (5, 20), (5, 21), (8, 33), (8, 64), (9, 43), (12, 14), (13, 34), (16, 24),
+                                 (17, 9), (20, 64), (28, 19), (32, 6), (32, 17), (32, 64)])
 def test_moments(hip, D, K, N, blocks):
     print(f"case gmm exact steps N={N} D={D} K={K} blocks={blocks}", flush=True)
     rng = np.random.default_rng(N + 100 * D + K)
