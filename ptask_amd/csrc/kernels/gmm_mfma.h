@@ -258,11 +258,7 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
             const int np = (int)min((long long)GMM_GROUP, d.N - p0);  // valid points (<= 0: none)
             // ---- E-step
             float a1[NF], a2[NF];
-            // a point past the last, whose square may overflow, lies at the centre
-            if (__builtin_expect(D < NF || np < GMM_GROUP, 0)) {
-#pragma unroll
-                for (int i = 0; i < NF; ++i) xe[i] = f0 + i < D && l16 < np ? xe[i] : g[i];
-            }
+            if (DC == 1 && D < NF) xe[NF - 1] = g[NF - 1];  // no dimension of the point's (see f0)
 #pragma unroll
             for (int i = 0; i < NF; ++i) {
                 a1[i] = xe[i] - g[i];
@@ -306,12 +302,9 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
             gmm_row_sum4(sum);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float inv = 4 * l4 + r < np ? __builtin_amdgcn_rcpf(sum[r]) : 0.f;
+                const float inv = __builtin_amdgcn_rcpf(sum[r]);
 #pragma unroll
-                for (int kt = 0; kt < KT; ++kt) {
-                    e[kt][r] *= inv;
-                    w[kt] += e[kt][r];
-                }
+                for (int kt = 0; kt < KT; ++kt) e[kt][r] *= inv;
                 lse[r] = mx[r] + __builtin_amdgcn_logf(sum[r]);
             }
             {   // the sixteen lanes of a row hold the same four values: lane l16 = r adds point r's
@@ -319,12 +312,21 @@ __device__ __forceinline__ bool gmm_mfma_tiles(const float *__restrict__ X, cons
                 if (l16 < 4 && 4 * l4 + l16 < np) ll += (double)v;
             }
             // ---- M-step
+            // a point past the last, whose square may overflow, has responsibility 0 and lies at the centre
             if (__builtin_expect(np < GMM_GROUP, 0)) {
 #pragma unroll
-                for (int j = 0; j < NS; ++j)
+                for (int r = 0; r < 4; ++r)
+                    if (4 * l4 + r >= np) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) xm[j][r] = 4 * l4 + r < np ? xm[j][r] : gm[j];
+                        for (int kt = 0; kt < KT; ++kt) e[kt][r] = 0.f;
+#pragma unroll
+                        for (int j = 0; j < NS; ++j) xm[j][r] = gm[j];
+                    }
             }
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w[kt] += e[kt][r];
             float x1[NS][4], x2[NS][4];
 #pragma unroll
             for (int j = 0; j < NS; ++j)
