@@ -31,11 +31,11 @@
 //
 // Bound: the matrix cores (8 N D K flops per step; 32 cycles of a SIMD per product).  Two waves per
 // SIMD (at most 256 registers) cover each other's log-sum-exp, about a quarter of the products'
-// issue time at D = 32, K = 64.  Measured there with N = 2M, 768 blocks: 306 us per launch, median (328
+// issue time at D = 32, K = 64.  Measured there with N = 2M, 768 blocks: 304 us per launch on average (328
 // with the tiles on all 768 rows, 313 without the log-sum-exp's priority), 70% of the rate of a large
 // matrix product; 612 us when tiles of coordinates and responsibilities passed through
 // LDS between the products (four barriers a tile, an LDS read per operand).  N = 50,001, D = 16, K = 24
-// (one tile per block): 13.5 us, 27.8 before, when every block first built the operand in LDS.
+// (one tile per block): 13.1 us, 27.8 before, when every block first built the operand in LDS.
 #pragma once
 
 #include "gmm_body.h"
