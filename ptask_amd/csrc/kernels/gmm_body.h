@@ -95,6 +95,9 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
                                                      long long t1, long long tstep, GmmShared &sh) {
 // Tolerance-checked binary32 work: let the compiler fuse multiply-adds (the build default is off).
 #pragma clang fp contract(fast)
+    // Components per turn of the E-phase's loops.  A loop more than twice unrolled costs the M-phase of few
+    // jobs up to a tenth.
+    constexpr int kDist = MATRIX || NC <= 2 ? 2 : 1, kExp = MATRIX ? 8 : 2;
     float *sX = sh.sX, *sR = sh.sR;
     const int D = d.D, K = d.K, Dp = 4 * NC, nc = NC;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -172,7 +175,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         }
         if (MATRIX) __builtin_amdgcn_s_setprio(1);  // the other block's products fill the matrix cores
         float mx = -INFINITY;
-#pragma unroll(MATRIX || NC <= 2 ? 2 : 1)
+#pragma unroll kDist
         for (int k = k0; k < k1; ++k) {
             const float *__restrict__ tk = tab + 2 * k * Dp;
             float s0 = 0.f, s1 = 0.f;
@@ -195,7 +198,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
         __syncthreads();
         mx = fmaxf(sh.sMax[0][ep], sh.sMax[1][ep]);
         float sum = 0.f;
-#pragma unroll(MATRIX ? 8 : 2)
+#pragma unroll kExp
         for (int k = k0; k < k1; ++k) sum += __expf(sR[ep * RS + k] - mx);
         sh.sSum[eh][ep] = sum;
         __syncthreads();
@@ -210,7 +213,7 @@ __device__ __forceinline__ void gmm_accumulate_tiles(const float *__restrict__ X
             }
             if (lane == 0) sh.sNz[wv] = nz;
         } else {
-#pragma unroll(MATRIX ? 8 : 2)
+#pragma unroll kExp
             for (int k = k0; k < k1; ++k) sR[ep * RS + k] = valid ? __expf(sR[ep * RS + k] - tmp) : 0.f;
         }
         if (valid && eh == 0) ll += (double)tmp;
